@@ -596,6 +596,20 @@ def test_gqa_verify_mfma(B, T, nq, nkv, D, lens):
         assert (err <= bound).all(), (b, float((err / bound).max()))
 
 
+@pytest.mark.parametrize("B,T,nq,nkv,D,lens", [
+    (2, 257, 24, 4, 256, [0, 383]),  # four-wave blocks; a chunk with no history, a whole last key tile
+    (1, 517, 24, 4, 256, [1003]),  # four-wave blocks, ragged rows and keys
+    (6, 258, 24, 4, 256, [0, 1, 63, 64, 500, 777]),  # eight-wave blocks
+    (3, 345, 12, 4, 128, [31, 0, 95]),  # group of 3
+    (4, 270, 48, 8, 128, [5, 250, 64, 0]),  # eight-wave blocks
+    (2, 513, 24, 8, 64, [700, 11]),
+    (4, 700, 16, 4, 64, [0, 129, 4, 63])])  # eight-wave blocks
+def test_gqa_verify_mfma_flash(B, T, nq, nkv, D, lens):
+    """Prompt chunks large enough for the flash form (48 blocks of 256 query
+    rows, 96 at D = 64), same bound as test_gqa_verify_mfma."""
+    test_gqa_verify_mfma(B, T, nq, nkv, D, lens)
+
+
 # ----------------------------------------------------------------- deltanet
 def _deltanet_case(rng, B, nk, nv, dk, dv, Kc=4):
     kw, vw = nk * dk, nv * dv

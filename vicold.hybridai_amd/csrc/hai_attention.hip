@@ -944,66 +944,109 @@ __global__ __launch_bounds__(256) void gqa_mfma_combine_wave_kernel(uint16_t* __
 
 // ---------------------------------------------------------------------------
 // Prompt chunks: flash attention with a block's K / V tiles shared by its
-// waves.  Block = 4 waves x 32 query rows (one KV head, one sequence); each
-// wave walks every key its rows see, 64 keys per tile (two 32-key score tiles):
+// waves.  Block = W waves x 32 query rows (one KV head, one sequence); each
+// wave walks every key its rows see, 64 keys per staged tile in two halves of
+// 32:
 //   S^T = K Q^T  on v_mfma_f32_32x32x16_bf16 (K rows the A operand from LDS,
 //                Q^T the B operand held in registers for the whole kernel);
 //   online softmax per query (base 2, the running max moved only past the
 //                same slack as gqa_mfma_partial_kernel, P rounded to bf16);
-//   O^T += V^T P^T  (V^T staged transposed in LDS; the result tile of S^T is
-//                the B operand of this product as it stands, under the key
-//                order 4 lh + q % 4 + 8 (q / 4) of k slot q).
-// K reaches LDS by global -> LDS copies, 16-byte piece p of key row r at
-// slot (D / 8) r + (p ^ (r % 16)); V through registers, transposed 8 keys x 8
-// dims per thread.  One barrier per tile.  The gated output O / l *
-// sigmoid(gate) is written directly: no split partials and no merge pass.
-// Same tolerance mode as the matrix-core verify attention.
+//   O^T += V^T P^T  (the result tile of S^T is the B operand of this product
+//                as it stands, under the key order 4 lh + q % 4 + 8 (q / 4)
+//                of k slot q; V^T comes out of the V rows in LDS through the
+//                transposing reads ds_read_b64_tr_b16).
+// K and V rows both reach LDS by global -> LDS copies issued a whole tile
+// ahead.  The copies are inline assembly: the compiler cannot tell which of
+// the two stages a copy writes and would wait for all of them before the
+// next LDS read (s_waitcnt vmcnt(0) right behind the request, the memory
+// latency exposed once per tile); here one counted wait and one barrier per
+// tile cover them.  Row r of a stage holds its 16-byte piece p at position
+// p ^ swizzle(r), chosen so that the lanes of one read fall in distinct
+// banks.  The gated output O / l * sigmoid(gate) is written directly: no
+// split partials and no merge pass.  Same tolerance mode as the matrix-core
+// verify attention.
+// Bound by the matrix cores and LDS together: a 64-key tile is 64 MFMAs (2048
+// cycles of a SIMD's matrix core per wave) and 64 KB of operand reads per
+// wave (128 B per clock and CU), two waves per SIMD.  MI355X, D = 256, 8 x
+// 1024 rows over 8192 keys: 3750 -> 1390 us (1.11 PFLOP/s) against four waves
+// of one per SIMD with V transposed through registers and the copies' wait
+// exposed.
 // ---------------------------------------------------------------------------
-constexpr int kFaRows = 128;  // query rows per block
-constexpr int kFaKeys = 64;   // keys per tile (two 32-key score tiles)
+constexpr int kFaWaveRows = 32;  // query rows per wave
+constexpr int kFaKeys = 64;      // keys per staged tile (two halves of 32)
 
 template <int D>
 struct FaShape {
-    static constexpr int KP = D / 8;               // 16-byte pieces of a K row
-    static constexpr int K_SLOTS = kFaKeys * KP;   // K tile, 16-byte slots
-    static constexpr int VTR = kFaKeys + 8;        // V^T row: the tile's keys + 16-byte pad (bf16)
-    static constexpr int STAGE_BYTES = K_SLOTS * 16 + D * VTR * 2;
-    static constexpr int LDS_BYTES = 2 * STAGE_BYTES;
-    static constexpr int KCOPY = K_SLOTS / 256;    // copy instructions per thread and tile
-    static constexpr int NKK = D / 16;             // 16-dim k steps of S^T
-    static constexpr int NDT = D / 32;             // 32-dim tiles of O^T
-    static constexpr int NST = kFaKeys / 32;       // score tiles per key tile
+    static constexpr int KP = D / 8;                  // 16-byte pieces of a K / V row
+    static constexpr int ROW = 2 * D;                 // bytes of a staged row
+    static constexpr int TILE = kFaKeys * ROW;        // bytes of a staged K (or V) tile
+    static constexpr int STAGE = 2 * TILE;            // K tile, then V tile
+    static constexpr int LDS_BYTES = 2 * STAGE;
+    static constexpr int NKK = D / 16;                // 16-dim k steps of S^T
+    static constexpr int NDT = D / 32;                // 32-dim tiles of O^T
+    // 16-byte piece positions of a row: K is read 32 rows x one piece, V 8
+    // rows x 64 bytes at a time
+    static __device__ __forceinline__ int k_swz(int r) { return D == 64 ? (r >> 1) & 7 : r & 15; }
+    static __device__ __forceinline__ int v_swz(int r) { return D == 64 ? ((r >> 1) & 1) << 2 : (r & 3) << 2; }
 };
 
-template <int D>
-__global__ __launch_bounds__(256) void gqa_fa_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
-                                                     const uint16_t* __restrict__ gate, const uint16_t* kc,
-                                                     const uint16_t* vc, int64_t cap, int T, int nq, int nkv,
-                                                     const int32_t* lens, int len_add, float scale_log2) {
+// One global -> LDS copy of 16 bytes per lane, to lds + 16 * lane (the
+// hazard between the M0 write and the copy needs one wait state).
+__device__ __forceinline__ void fa_copy16(uint32_t off, const void* base, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(off), "s"(base), "s"(lds)
+                 : "memory");
+}
+__device__ __forceinline__ uint2 fa_read_tr(uint32_t lds) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4*)(uintptr_t)lds);
+    return __builtin_bit_cast(uint2, v);
+}
+__device__ __forceinline__ u32x4 fa_read16(uint32_t lds) {
+    return *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)lds;
+}
+
+// 1 / (1 + e^-x) by the hardware exp2 and reciprocal (tolerance mode).
+__device__ __forceinline__ float fast_sigmoid(float x) {
+    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
+}
+
+template <int D, int W>
+__global__ __launch_bounds__(64 * W) void gqa_fa_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
+                                                        const uint16_t* __restrict__ gate, const uint16_t* kc,
+                                                        const uint16_t* vc, int64_t cap, int T, int nq, int nkv,
+                                                        const int32_t* lens, int len_add, float scale_log2) {
     using S = FaShape<D>;
-    constexpr int NST = S::NST;
-    static_assert(D % 32 == 0 && S::K_SLOTS % 256 == 0 && kFaKeys % 32 == 0, "tile shapes");
+    constexpr int ROWS = kFaWaveRows * W;
+    constexpr int COPIES = S::TILE / (1024 * W);     // copies per thread for K (and for V)
+    constexpr int COPY_ROWS = 1024 * W / S::ROW;     // rows between a thread's copies
+    static_assert(COPIES >= 1 && COPY_ROWS % 4 == 0, "copies per thread");
     constexpr float kNegInf = -__builtin_huge_valf();
-    extern __shared__ __align__(16) unsigned char fa_lds[];
-    const int qblk = blockIdx.x;
+    extern __shared__ __align__(1024) unsigned char fa_lds[];
+    // the blocks with the most visible keys first
+    const int qblk = gridDim.x - 1 - blockIdx.x;
     const int kvh = blockIdx.y;
     const int b = blockIdx.z;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
+    const int lane = threadIdx.x & 63;
     const int wave = wave_index();
     const int lc = lane & 31;
     const int lh = lane >> 5;
     const int group = nq / nkv;
     const int nqry = T * group;
-    const int64_t L = static_cast<int64_t>(lens ? lens[b] : 0) + len_add;
-    const int q0 = qblk * kFaRows;
+    const int L = __builtin_amdgcn_readfirstlane((lens ? lens[b] : 0) + len_add);
+    const int q0 = qblk * ROWS;
+    const int w0 = q0 + kFaWaveRows * wave;
     // the lane's query (padding rows past nqry take the last token and are not stored)
-    const int qi = q0 + 32 * wave + lc;
+    const int qi = w0 + lc;
     const int tq = qi < nqry ? qi / group : T - 1;
-    const int64_t lim = L - T + tq + 1;  // keys [0, lim) are visible
-    const int t_last = (min(q0 + kFaRows, nqry) - 1) / group;
-    const int64_t nkeys = L - T + t_last + 1;  // keys any query of the block sees
-    const int ntiles = static_cast<int>((nkeys + kFaKeys - 1) / kFaKeys);
+    const int lim = L - T + tq + 1;  // keys [0, lim) are visible
+    // the fewest / most keys a query of this wave sees, and the most of the block
+    const int lim_lo = __builtin_amdgcn_readfirstlane(L - T + min(w0 / group, T - 1) + 1);
+    const int lim_hi = __builtin_amdgcn_readfirstlane(L - T + min((w0 + kFaWaveRows - 1) / group, T - 1) + 1);
+    const int nkeys = L - T + min((q0 + ROWS - 1) / group, T - 1) + 1;
+    const int ntiles = (nkeys + kFaKeys - 1) / kFaKeys;
 
     // Q^T operand: k step kk holds dims 16 kk + 8 lh + [0, 8) of the lane's query
     u32x4 qr[S::NKK];
@@ -1014,48 +1057,39 @@ __global__ __launch_bounds__(256) void gqa_fa_kernel(uint16_t* __restrict__ out,
         for (int kk = 0; kk < S::NKK; ++kk) qr[kk] = *reinterpret_cast<const u32x4*>(qp + 16 * kk);
     }
 
-    const uint16_t* kbase = kc + (static_cast<int64_t>(b) * cap * nkv + kvh) * D;
-    const uint16_t* vbase = vc + (static_cast<int64_t>(b) * cap * nkv + kvh) * D;
-    const int64_t kstride = static_cast<int64_t>(nkv) * D;  // elements between consecutive keys
-    auto key_row = [&](int64_t key) { return min(key, L - 1) * kstride; };  // keys past L: the last row (masked)
-    // K copies: instruction i of this wave covers slots (4 i + wave) * 64 + lane
-    auto copy_k = [&](int tile, int buf) {
-        u32x4* dst = reinterpret_cast<u32x4*>(fa_lds + buf * S::STAGE_BYTES);
+    const uint32_t lds0 = static_cast<uint32_t>(
+        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)fa_lds));
+    // copies: thread slot s = 64 (W i + wave) + lane of a tile is row s / KP
+    // (rows COPY_ROWS apart for consecutive i), position s % KP
+    const uint32_t kstride = static_cast<uint32_t>(nkv) * D * 2u;  // bytes between consecutive keys
+    const int64_t head = (static_cast<int64_t>(b) * cap * nkv + kvh) * D;
+    const int crow = (64 * wave + lane) / S::KP;
+    const int cpos = lane % S::KP;
+    auto kpiece = [&](int i) {  // (one value for every i when the rows are 16 apart)
+        return static_cast<uint32_t>(cpos ^ S::k_swz(COPY_ROWS % 16 == 0 ? crow : crow + COPY_ROWS * i)) * 16u;
+    };
+    const uint32_t vpiece = static_cast<uint32_t>(cpos ^ S::v_swz(crow)) * 16u;
+    auto copy_tile = [&](int tile, int buf) {
+        const int k0 = tile * kFaKeys;
+        const int64_t at = (head + static_cast<int64_t>(k0) * nkv * D) * 2;
+        const char* kb = reinterpret_cast<const char*>(kc) + at;
+        const char* vb = reinterpret_cast<const char*>(vc) + at;
+        const int last = L - 1 - k0;  // rows past the cache: its last row (masked)
+        const uint32_t dst = lds0 + static_cast<uint32_t>(buf * S::STAGE + wave * 1024);
 #pragma unroll
-        for (int i = 0; i < S::KCOPY; ++i) {
-            const int s = (4 * i + wave) * 64 + lane;
-            const int r = s / S::KP, p = (s % S::KP) ^ (r & 15);
-            const uint16_t* src = kbase + key_row(static_cast<int64_t>(tile) * kFaKeys + r) + 8 * p;
-            __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)(dst + (4 * i + wave) * 64),
-                                             16, 0, 0);
+        for (int i = 0; i < COPIES; ++i) {
+            const uint32_t ro = static_cast<uint32_t>(min(crow + COPY_ROWS * i, last)) * kstride;
+            fa_copy16(ro + kpiece(i), kb, dst + i * W * 1024);
+            fa_copy16(ro + vpiece, vb, dst + S::TILE + i * W * 1024);
         }
     };
-    // V: thread (kq = tid / (D / 8), dp = tid % (D / 8)) loads keys VK kq + [0, VK) x dims 8 dp + [0, 8)
-    constexpr int VT_DIMS = D / 8;
-    constexpr int VK = kFaKeys * VT_DIMS / 256;  // keys per thread (8 at D = 256)
-    static_assert(VK == 4 || VK == 8, "V block per thread");
-    const int vkq = tid / VT_DIMS, vdp = tid % VT_DIMS;
-    u32x4 vr[VK];
-    auto load_v = [&](int tile) {
-#pragma unroll
-        for (int i = 0; i < VK; ++i)
-            vr[i] = *reinterpret_cast<const u32x4*>(
-                vbase + key_row(static_cast<int64_t>(tile) * kFaKeys + VK * vkq + i) + 8 * vdp);
-    };
-    auto stage_v = [&](int buf) {
-        uint16_t* vt = reinterpret_cast<uint16_t*>(fa_lds + buf * S::STAGE_BYTES + S::K_SLOTS * 16);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            // keys VK kq .. VK kq + VK - 1 of dim 8 dp + j
-            const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
-            uint32_t d[VK / 2];
-#pragma unroll
-            for (int w = 0; w < VK / 2; ++w) d[w] = __builtin_amdgcn_perm(vr[2 * w + 1][j >> 1], vr[2 * w][j >> 1], sel);
-            uint16_t* dst = vt + (8 * vdp + j) * S::VTR + VK * vkq;
-            if constexpr (VK == 8) *reinterpret_cast<u32x4*>(dst) = u32x4{d[0], d[1], d[2], d[3]};
-            else *reinterpret_cast<uint2*>(dst) = make_uint2(d[0], d[1]);
-        }
-    };
+    // K operand of k step kk: piece 2 kk + lh of row lc (+ 32 per half)
+    const uint32_t ka0 = lds0 + lc * S::ROW + ((lh ^ S::k_swz(lc)) << 4);
+    // V^T operand of dims 32 dt + lc: rows 4 lh + (li / 4), 8-byte piece li % 4 of the 16 dims of the lane's 16-group
+    const int li = lane & 15;
+    const uint32_t va0 = lds0 + S::TILE + (4 * lh + (li >> 2)) * S::ROW +
+                         (((2 * ((lane >> 4) & 1) + ((li & 3) >> 1)) ^ S::v_swz(4 * lh + (li >> 2))) << 4) +
+                         ((li & 1) << 3);
 
     float m = kNegInf, l = 0.0f;
     f32x16 o[S::NDT];
@@ -1064,94 +1098,104 @@ __global__ __launch_bounds__(256) void gqa_fa_kernel(uint16_t* __restrict__ out,
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
 
-    if (ntiles > 0) {
-        copy_k(0, 0);
-        load_v(0);
-        stage_v(0);
-    }
-    __syncthreads();
-    const int ksw = lc & 15;  // swizzle of the lane's K rows
+    if (ntiles > 0) copy_tile(0, 0);
     for (int j = 0; j < ntiles; ++j) {
         const int buf = j & 1;
-        if (j + 1 < ntiles) {
-            copy_k(j + 1, buf ^ 1);
-            load_v(j + 1);
-        }
-        const u32x4* ks = reinterpret_cast<const u32x4*>(fa_lds + buf * S::STAGE_BYTES);
-        const uint16_t* vt = reinterpret_cast<const uint16_t*>(fa_lds + buf * S::STAGE_BYTES + S::K_SLOTS * 16);
-        // ---- S^T = K Q^T per 32-key score tile t: row = key 32 t + 8 (i / 4) + 4 lh + i % 4, column = the
-        // lane's query; the tiles' chains interleaved ----
-        f32x16 st[NST];
+        wait_vmcnt<0>();  // this wave's copies of tile j have landed ...
+        lds_barrier();    // ... and every wave's; the other stage is free
+        if (j + 1 < ntiles) copy_tile(j + 1, buf ^ 1);
 #pragma unroll
-        for (int t = 0; t < NST; ++t)
+        for (int h = 0; h < 2; ++h) {
+            const int k0 = j * kFaKeys + 32 * h;
+            if (k0 >= lim_hi) break;  // no query of this wave sees this half or a later one
+            const uint32_t ka = ka0 + buf * S::STAGE + h * 32 * S::ROW;
+            const uint32_t va = va0 + buf * S::STAGE + h * 32 * S::ROW;
+            // ---- S^T = K Q^T: row = key 8 (i / 4) + 4 lh + i % 4, column = the lane's query; the operands
+            // of the next kG k steps are read while those of the last kG are multiplied ----
+            constexpr int kG = 2;
+            f32x16 st;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) st[t][i] = 0.0f;
+            for (int i = 0; i < 16; ++i) st[i] = 0.0f;
+            u32x4 kf[2][kG];
 #pragma unroll
-        for (int kk = 0; kk < S::NKK; ++kk)
+            for (int e = 0; e < kG; ++e) kf[0][e] = fa_read16(ka ^ (e << 5));
 #pragma unroll
-            for (int t = 0; t < NST; ++t) {
-                const u32x4 ka = ks[(32 * t + lc) * S::KP + ((2 * kk + lh) ^ ksw)];
-                st[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ka),
-                                                               __builtin_bit_cast(bf16x8, qr[kk]), st[t], 0, 0, 0);
+            for (int g = 0; g < S::NKK / kG; ++g) {
+                if (g + 1 < S::NKK / kG)
+#pragma unroll
+                    for (int e = 0; e < kG; ++e) kf[(g + 1) & 1][e] = fa_read16(ka ^ (((g + 1) * kG + e) << 5));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < kG; ++e)
+                    st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[g & 1][e]),
+                                                                 __builtin_bit_cast(bf16x8, qr[g * kG + e]), st, 0, 0,
+                                                                 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
-        // ---- online softmax of the lane's query over the tile ----
-        const int64_t k0 = static_cast<int64_t>(j) * kFaKeys;
-        float mx = kNegInf;
+            // the first V^T operands on their way during the softmax
+            constexpr int kV = 2;  // operands per group
+            constexpr int NV = 2 * S::NDT;
+            auto read_v = [&](int n) {  // operand n: 16-key step n / NDT, dims 32 (n % NDT)
+                const uint32_t at = (va ^ ((n % S::NDT) << 6)) + (n / S::NDT) * 16 * S::ROW;
+                const uint2 lo = fa_read_tr(at), hi = fa_read_tr(at + 8 * S::ROW);
+                return u32x4{lo.x, lo.y, hi.x, hi.y};
+            };
+            u32x4 vf[2][kV];
 #pragma unroll
-        for (int t = 0; t < NST; ++t)
+            for (int e = 0; e < kV; ++e) vf[0][e] = read_v(e);
+            // ---- online softmax of the lane's query over the half (scores in base 2 units) ----
+            if (k0 + 32 > lim_lo) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (k0 + 8 * (i >> 2) + 4 * lh + (i & 3) >= lim) st[i] = kNegInf;
+            }
+            float mx = fmaxf(st[0], st[1]);
+#pragma unroll
+            for (int i = 2; i < 16; ++i) mx = fmaxf(mx, st[i]);
+            mx = fmaxf(mx, __shfl_xor(mx, 32)) * scale_log2;
+            const bool grow = mx > m + kRescaleSlack;  // true for the first visible key
+            if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+                const float mn = grow ? mx : m;
+                const float alpha = grow ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;  // 0 from -inf
+                l *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < S::NDT; ++dt) o[dt] *= alpha;
+                m = mn;
+            }
+            const float sub = m == kNegInf ? 0.0f : -m;  // no visible key yet: every p is 0
+            float ps[2] = {0.0f, 0.0f};
+            bf16x8 pb[2];
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const int64_t key = k0 + 32 * t + 8 * (i >> 2) + 4 * lh + (i & 3);
-                const float x = key < lim ? st[t][i] * scale_log2 : kNegInf;
-                st[t][i] = x;
-                mx = fmaxf(mx, x);
+                const float p = __builtin_amdgcn_exp2f(fma_(st[i], scale_log2, sub));
+                ps[i & 1] += p;
+                pb[i >> 3][i & 7] = static_cast<__bf16>(p);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const bool grow = mx > m + kRescaleSlack;  // true for the first visible key
-        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-            const float mn = grow ? mx : m;
-            const float alpha = grow ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;  // 0 from -inf
-            l *= alpha;
+            l += ps[0] + ps[1];
+            // ---- O^T += V^T P^T: k step s covers keys 16 s + (4 lh + q % 4 + 8 (q / 4)), q the k slot ----
 #pragma unroll
-            for (int dt = 0; dt < S::NDT; ++dt) o[dt] *= alpha;
-            m = mn;
-        }
-        const float sub = m == kNegInf ? 0.0f : m;  // no visible key yet: every p is 0
-        float ps = 0.0f;
+            for (int g = 0; g < NV / kV; ++g) {
+                if (g + 1 < NV / kV)
 #pragma unroll
-        for (int t = 0; t < NST; ++t)
+                    for (int e = 0; e < kV; ++e) vf[(g + 1) & 1][e] = read_v((g + 1) * kV + e);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float p = __builtin_amdgcn_exp2f(st[t][i] - sub);
-                st[t][i] = p;
-                ps += p;
-            }
-        l += ps;
-        // ---- O^T += V^T P^T: k step s covers keys 16 s + (4 lh + q % 4 + 8 (q / 4)), q the k slot ----
-#pragma unroll
-        for (int s = 0; s < 2 * NST; ++s) {
-            const f32x16& sp = st[s >> 1];
-            const int e = 8 * (s & 1);
-            const bf16x8 pb = bf16x8{static_cast<__bf16>(sp[e]), static_cast<__bf16>(sp[e + 1]),
-                                     static_cast<__bf16>(sp[e + 2]), static_cast<__bf16>(sp[e + 3]),
-                                     static_cast<__bf16>(sp[e + 4]), static_cast<__bf16>(sp[e + 5]),
-                                     static_cast<__bf16>(sp[e + 6]), static_cast<__bf16>(sp[e + 7])};
-#pragma unroll
-            for (int dt = 0; dt < S::NDT; ++dt) {
-                const uint16_t* vrow = vt + (32 * dt + lc) * S::VTR + 16 * s + 4 * lh;
-                const uint2 lo = *reinterpret_cast<const uint2*>(vrow);
-                const uint2 hi = *reinterpret_cast<const uint2*>(vrow + 8);
-                const u32x4 va = u32x4{lo.x, lo.y, hi.x, hi.y};
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va), pb, o[dt], 0, 0, 0);
+                for (int e = 0; e < kV; ++e) {
+                    const int n = g * kV + e;
+                    o[n % S::NDT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[g & 1][e]),
+                                                                            pb[n / S::NDT], o[n % S::NDT], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (j + 1 < ntiles) stage_v(buf ^ 1);
-        __syncthreads();  // the next tile is staged; this tile's buffer is free
     }
 
-    // ---- O / l * sigmoid(gate), rounded: lane holds dims 32 dt + 8 (i / 4) + 4 lh + i % 4 ----
+    // ---- O / l * sigmoid(gate), rounded: lane holds dims 32 dt + 8 (i / 4) + 4 lh + i % 4.  One reciprocal
+    // per query and the hardware exp2 / reciprocal (fp32, 1 ulp) for the gate: D / 2 IEEE divisions and
+    // canonical exps per lane were a third of the kernel's time at 1024 x 1024 ----
     if (qi >= nqry) return;
     l += __shfl_xor(l, 32);
+    const float inv = 1.0f / l;
     const int64_t row = (static_cast<int64_t>(b) * T + tq) * nq + kvh * group + qi % group;
 #pragma unroll
     for (int dt = 0; dt < S::NDT; ++dt)
@@ -1160,13 +1204,13 @@ __global__ __launch_bounds__(256) void gqa_fa_kernel(uint16_t* __restrict__ out,
             const int d = 32 * dt + 8 * g4 + 4 * lh;
             float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = o[dt][4 * g4 + e] / l;
+            for (int e = 0; e < 4; ++e) v[e] = o[dt][4 * g4 + e] * inv;
             if (gate != nullptr) {
                 const uint2 gv = *reinterpret_cast<const uint2*>(gate + row * D + d);
-                v[0] *= csigmoid(lo_bf(gv.x));
-                v[1] *= csigmoid(hi_bf(gv.x));
-                v[2] *= csigmoid(lo_bf(gv.y));
-                v[3] *= csigmoid(hi_bf(gv.y));
+                v[0] *= fast_sigmoid(lo_bf(gv.x));
+                v[1] *= fast_sigmoid(hi_bf(gv.x));
+                v[2] *= fast_sigmoid(lo_bf(gv.y));
+                v[3] *= fast_sigmoid(hi_bf(gv.y));
             }
             *reinterpret_cast<uint2*>(out + row * D + d) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
         }
@@ -1186,7 +1230,7 @@ inline int attn_device_cus() {
     return 256;  // MI355X
 }
 
-// The flash form for prompt chunks (HAI_ATTN_FA=0, read once per process,
+// The flash form for prompt chunks, see fa_waves (HAI_ATTN_FA=0, read once per process,
 // keeps the split form for every shape).
 inline bool fa_enabled() {
     static const bool on = [] {
@@ -1194,6 +1238,30 @@ inline bool fa_enabled() {
         return e == nullptr || e[0] != '0';
     }();
     return on;
+}
+
+// Waves per block of the flash form for these calls, 0 for the split form.
+// The flash form reads every K / V tile once per 32 W query rows and needs
+// no merge pass, but a block walks its whole key range alone (2.8 us per 64
+// keys at D = 256), so it needs enough blocks; the split form spreads the
+// keys of few rows over the device.  Measured on MI355X (us, split / flash),
+// blocks counted at 256 rows: D = 256, 1 x 512 rows over 512 / 8192 keys (48
+// blocks) 52 / 38 and 405 / 348, 1 x 1024 over 1024 (96) 100 / 60, 4 x 1024
+// over 4096 (384) 1413 / 428, against 46 / 58 at 32 blocks; D = 128 76 / 117
+// at 24 blocks, 105 / 64 at 48, 433 / 231 at 128; D = 64 143 / 165 at 64,
+// 37 / 28 and 172 / 165 at 96.  Below half the CUs four-wave blocks (twice as
+// many) are 5-15 % faster; from there on eight waves are (2 x 1024 over 1024,
+// 192 blocks: 102 / 69), two per SIMD covering each other's softmax and LDS
+// latency.  128 rows at least: fewer leave the block's other rows idle.
+// The output and gate rows are accessed 8 bytes at a time.
+inline int fa_waves(int D, int64_t B, int64_t nqry, int64_t nkv, const void* out, const void* gate) {
+    if (!fa_enabled() || nqry < 128 || nkv * D > (1 << 24)) return 0;
+    if (((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(gate)) & 7u) != 0) return 0;
+    const int64_t cus = attn_device_cus();
+    const int64_t rows = nqry * nkv * B;
+    const int64_t blocks = (nqry + 255) / 256 * nkv * B;
+    if (rows < (D == 64 ? 96 * cus : 48 * cus)) return 0;  // 3/8 (3/16) of the CUs x 256 rows
+    return 2 * blocks <= cus ? 4 : 8;
 }
 
 // Split plan of the matrix-core path: steps per wave (block = 4 waves x steps
@@ -1223,35 +1291,36 @@ inline MfmaPlan mfma_plan(int D, int64_t B, int64_t T, int64_t nq, int64_t nkv, 
     return p;
 }
 
+template <int D, int W>
+int launch_fa(uint16_t* out, const uint16_t* q, const uint16_t* gate, const uint16_t* kc, const uint16_t* vc,
+              int64_t cap, int B, int T, int nq, int nkv, const int32_t* lens, int len_add, hipStream_t s) {
+    constexpr size_t shmem = FaShape<D>::LDS_BYTES;
+    static std::atomic<uint8_t> allowed[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return invalid("gqa_verify_mfma: device");
+    if (!allowed[dev].load(std::memory_order_acquire)) {
+        const int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(gqa_fa_kernel<D, W>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     static_cast<int>(shmem)),
+                                 "hipFuncSetAttribute");
+        if (rc != HAI_OK) return rc;
+        allowed[dev].store(1, std::memory_order_release);
+    }
+    const int64_t nqry = static_cast<int64_t>(T) * (nq / nkv);
+    const dim3 grid(static_cast<unsigned>((nqry + kFaWaveRows * W - 1) / (kFaWaveRows * W)), nkv, B);
+    const float sl2 = 1.4426950408889634f / __builtin_sqrtf(static_cast<float>(D));
+    gqa_fa_kernel<D, W><<<grid, dim3(64 * W), shmem, s>>>(out, q, gate, kc, vc, cap, T, nq, nkv, lens, len_add, sl2);
+    return launched("gqa_fa_kernel");
+}
+
 template <int D>
 int launch_mfma(uint16_t* out, const uint16_t* q, const uint16_t* gate, const uint16_t* kc, const uint16_t* vc,
                 int64_t cap, float* scratch, int B, int T, int nq, int nkv, const int32_t* lens, int len_add,
                 int64_t max_len, hipStream_t s) {
     const int64_t nqry = static_cast<int64_t>(T) * (nq / nkv);
-    if constexpr (D == 256) {
-        // prompt chunks: whole key ranges per block of 128 query rows, when
-        // those blocks fill the device (fewer, and the split form's key
-        // splits spread the work wider: 1 x 1024 rows 105 against 111 us)
-        constexpr size_t shmem = FaShape<D>::LDS_BYTES;
-        const int64_t fa_blocks = (nqry + kFaRows - 1) / kFaRows * nkv * B;
-        if (nqry >= kFaRows && fa_enabled() && fa_blocks >= attn_device_cus()) {
-            static std::atomic<uint8_t> allowed[64];
-            int dev = 0;
-            if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return invalid("gqa_verify_mfma: device");
-            if (!allowed[dev].load(std::memory_order_acquire)) {
-                const int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(gqa_fa_kernel<D>),
-                                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                             static_cast<int>(shmem)),
-                                         "hipFuncSetAttribute");
-                if (rc != HAI_OK) return rc;
-                allowed[dev].store(1, std::memory_order_release);
-            }
-            const dim3 grid(static_cast<unsigned>((nqry + kFaRows - 1) / kFaRows), nkv, B);
-            const float sl2 = 1.4426950408889634f / __builtin_sqrtf(static_cast<float>(D));
-            gqa_fa_kernel<D><<<grid, dim3(256), shmem, s>>>(out, q, gate, kc, vc, cap, T, nq, nkv, lens, len_add, sl2);
-            return launched("gqa_fa_kernel");
-        }
-    }
+    if (const int w = fa_waves(D, B, nqry, nkv, out, gate); w != 0)
+        return w == 8 ? launch_fa<D, 8>(out, q, gate, kc, vc, cap, B, T, nq, nkv, lens, len_add, s)
+                      : launch_fa<D, 4>(out, q, gate, kc, vc, cap, B, T, nq, nkv, lens, len_add, s);
     const void* kern = nqry <= 16 ? reinterpret_cast<const void*>(gqa_mfma_partial_kernel<D, 1>)
                                   : reinterpret_cast<const void*>(gqa_mfma_partial_kernel<D, 2>);
     const int64_t resident = resident_blocks(kern, 0);
