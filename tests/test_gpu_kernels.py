@@ -452,6 +452,18 @@ def test_qkv_norm_rope_append_equals_the_two_launches(B, T, nq, nkv, D, R):
         assert np.array_equal(a, b), name
 
 
+@pytest.mark.parametrize("B,T,nq,nkv,D,R", [
+    (2, 3, 3, 1, 96, 32),  # 12 of a row's 16 lanes hold dims
+    (1, 5, 7, 1, 40, 16),  # 5 of 8, a ragged last block
+    (1, 2, 4, 2, 512, 64),  # one row per wave
+    (1, 2, 4, 2, 256, 256),  # every dim rotated
+    (1, 3, 4, 2, 64, 12)])  # R / 2 not a multiple of 8: the two-byte form
+def test_qkv_norm_rope_append_row_forms(B, T, nq, nkv, D, R):
+    """Both forms of the fused launch (16-byte stores with several rows per
+    wave, two-byte stores) against the q/gate and K/V launches, bit for bit."""
+    test_qkv_norm_rope_append_equals_the_two_launches(B, T, nq, nkv, D, R)
+
+
 @pytest.mark.parametrize("B,T,nq,nkv,D,R,L0", [
     (1, 2, 24, 4, 256, 64, [1278]),       # C3 verify: both new rows in the last chunk
     (1, 2, 24, 4, 256, 64, [63]),         # new rows straddle chunks 0 and 1

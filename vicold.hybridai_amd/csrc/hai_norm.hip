@@ -189,6 +189,88 @@ __global__ __launch_bounds__(256) void qkv_rmsnorm_rope_append_kernel(QkvNormArg
     }
 }
 
+// The same rows with 16-byte stores and no LDS: LPH lanes own a head row (8
+// dims each, a wave takes 64 / LPH rows), the rotation partners come from the
+// lane R / 16 away.  Same bits: the lanes past a row's D / 8 hold zeros, as
+// the lanes of l64_sumsq_bf16's butterfly past it do, so the butterfly over
+// LPH lanes gives the sum of the one over 64.  Needs R / 2 a multiple of 8
+// and every pointer 16-byte aligned.  Bound by memory traffic (the rows read
+// and written once): the kernel above stores two bytes per lane, the gate and
+// V rows 16 bytes apart (MI355X, 8192 rows of 24 + 4 heads x 256: 178 -> 79
+// us, 5.9 TB/s).
+template <int LPH>
+__device__ __forceinline__ float group_sum(float v) {
+#pragma unroll
+    for (int s = LPH / 2; s >= 4; s >>= 1) v = v + __shfl_xor(v, s, 64);
+    v = v + quad_xor2(v);
+    return v + quad_xor1(v);
+}
+template <int LPH>
+__global__ __launch_bounds__(256) void qkv_rmsnorm_rope_append_vec_kernel(QkvNormArgs a) {
+    const int lane = threadIdx.x & (LPH - 1);
+    constexpr int ROWS = 256 / LPH;  // head rows per block
+    const bool is_q = static_cast<int>(blockIdx.x) < a.qblocks;
+    const int64_t pair = static_cast<int64_t>(is_q ? blockIdx.x : blockIdx.x - a.qblocks) * ROWS + threadIdx.x / LPH;
+    const int heads = is_q ? a.nq : a.nkv;
+    const int64_t m = pair / heads;
+    const int h = static_cast<int>(pair % heads);
+    const bool row = m < static_cast<int64_t>(a.B) * a.T;
+    const bool active = row && lane * 8 < a.D;
+    const int half = a.R / 2;
+    const int d0 = lane * 8;
+    const bool rotated = active && d0 < a.R;
+    u32x4 xd = {0u, 0u, 0u, 0u}, cd = {0u, 0u, 0u, 0u}, wd = {0u, 0u, 0u, 0u};
+    const int b = row ? static_cast<int>(m / a.T) : 0;
+    const int t = row ? static_cast<int>(m % a.T) : 0;
+    if (active) {
+        // q: [q_h | gate_h]; k: the K head, then its V head behind all K heads
+        const uint16_t* s = a.src + m * a.ld_src + (is_q ? static_cast<int64_t>(h) * 2 : 2 * a.nq + h) * a.D + d0;
+        xd = *reinterpret_cast<const u32x4*>(s);
+        cd = *reinterpret_cast<const u32x4*>(s + (is_q ? a.D : static_cast<int64_t>(a.nkv) * a.D));
+        wd = *reinterpret_cast<const u32x4*>((is_q ? a.wq : a.wk) + d0);
+    }
+    const int64_t pos = static_cast<int64_t>(a.lens ? a.lens[b] : 0) + a.pos_add + t;
+    float c[8], sn[8];
+    if (rotated) {
+        const int64_t rp = pos < 0 ? 0 : (pos >= a.rope_pos ? a.rope_pos - 1 : pos);
+        const int64_t at = rp * half + (d0 < half ? d0 : d0 - half);
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            *reinterpret_cast<float4*>(c + e) = *reinterpret_cast<const float4*>(a.rc + at + e);
+            *reinterpret_cast<float4*>(sn + e) = *reinterpret_cast<const float4*>(a.rs + at + e);
+        }
+    }
+    float acc = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        acc = fma_(lo_bf(xd[q]), lo_bf(xd[q]), acc);
+        acc = fma_(hi_bf(xd[q]), hi_bf(xd[q]), acc);
+    }
+    const float inv = 1.0f / csqrt(group_sum<LPH>(acc) / static_cast<float>(a.D) + a.eps);
+    float v[8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        v[2 * q] = (lo_bf(xd[q]) * inv) * (lo_bf(wd[q]) + 1.0f);
+        v[2 * q + 1] = (hi_bf(xd[q]) * inv) * (hi_bf(wd[q]) + 1.0f);
+    }
+    if (!is_q) {  // K is stored once before the rotation
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = bfr(v[e]);
+    }
+    const int partner = (threadIdx.x & 63) + (d0 < half ? half / 8 : -(half / 8));
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float pv = __shfl(v[e], partner, 64);
+        o[e] = !rotated ? v[e] : d0 < half ? fma_(v[e], c[e], -(pv * sn[e])) : fma_(v[e], c[e], pv * sn[e]);
+    }
+    if (!active || (!is_q && (pos < 0 || pos >= a.cap))) return;
+    const int64_t dst = (is_q ? m * a.nq + h : (static_cast<int64_t>(b) * a.cap + pos) * a.nkv + h) * a.D + d0;
+    *reinterpret_cast<u32x4*>((is_q ? a.q_out : a.kc) + dst) =
+        u32x4{f2bf2(o[0], o[1]), f2bf2(o[2], o[3]), f2bf2(o[4], o[5]), f2bf2(o[6], o[7])};
+    *reinterpret_cast<u32x4*>((is_q ? a.g_out : a.vc) + dst) = cd;
+}
+
 __global__ void append_kv_kernel(uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int64_t cap,
                                  const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int B,
                                  int T, int64_t row_width, const int32_t* lens, int pos_add) {
@@ -423,6 +505,20 @@ int hai_qkv_rmsnorm_rope_append_bf16(void* q_out, void* gate_out, void* k_cache,
     a.pos_add = pos_add;
     a.qblocks = int((qpairs + 3) / 4);
     a.eps = eps;
+    if ((a.R / 2) % 8 == 0 && aligned16(q_out) && aligned16(gate_out) && aligned16(k_cache) && aligned16(v_cache) &&
+        aligned16(q_norm) && aligned16(k_norm) && aligned16(rope_cos) && aligned16(rope_sin)) {
+        auto vec = [&](auto kern, int lph) {
+            const int64_t rows = 256 / lph;
+            a.qblocks = int((qpairs + rows - 1) / rows);
+            const unsigned blocks = static_cast<unsigned>(a.qblocks + (kvpairs + rows - 1) / rows);
+            kern<<<dim3(blocks), dim3(256), 0, as_stream(stream)>>>(a);
+            return launched("qkv_rmsnorm_rope_append_vec_kernel");
+        };
+        if (D <= 64) return vec(qkv_rmsnorm_rope_append_vec_kernel<8>, 8);
+        if (D <= 128) return vec(qkv_rmsnorm_rope_append_vec_kernel<16>, 16);
+        if (D <= 256) return vec(qkv_rmsnorm_rope_append_vec_kernel<32>, 32);
+        return vec(qkv_rmsnorm_rope_append_vec_kernel<64>, 64);
+    }
     const unsigned blocks = static_cast<unsigned>(a.qblocks + (kvpairs + 3) / 4);
     qkv_rmsnorm_rope_append_kernel<<<dim3(blocks), dim3(256), 0, as_stream(stream)>>>(a);
     return launched("qkv_rmsnorm_rope_append_kernel");
