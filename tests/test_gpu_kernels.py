@@ -848,6 +848,17 @@ def test_deltanet_prefill_against_oracle(nk, nv, dk, T, Kc):
             assert np.array_equal(ring_got[b, pos % ring], pb.reshape(B, T, width)[b, T - hist + i, :C]), (b, i)
 
 
+@pytest.mark.parametrize("nk,nv,dk,T,Kc", [
+    (8, 72, 128, 45, 4),  # 144 heads: a head's value columns on one block
+    (1, 3, 128, 65, 4),  # on two; a last chunk of one token
+    (4, 4, 64, 3, 4),  # as many tokens as conv history
+    (2, 2, 128, 33, 3)])  # projection rows not a multiple of 16 bytes: the gated norm's two-byte form
+def test_deltanet_prefill_forms(nk, nv, dk, T, Kc):
+    """The forms of the state pass and of the gated norm, and the edges of
+    their chunks, same bound as test_deltanet_prefill_against_oracle."""
+    test_deltanet_prefill_against_oracle(nk, nv, dk, T, Kc)
+
+
 @pytest.mark.parametrize("B,nk,nv,dk,T,Kc,ab", [(3, 2, 6, 64, 40, 4, False), (2, 16, 48, 128, 33, 4, True),
                                                 (1, 4, 4, 64, 100, 3, False)])
 def test_deltanet_prompt_chunk_equals_16_token_launches(B, nk, nv, dk, T, Kc, ab):
