@@ -1408,6 +1408,52 @@ def test_gemm_fp8_mfma_within_tolerance(M, N, K, epi, mapped, special):
     assert np.allclose(got, want, rtol=2 ** -6, atol=2e-3 * scale), float(np.abs(got - want).max())
 
 
+@pytest.mark.parametrize("fp8,M,N,K,epi,mapped", [
+    (True, 1, 33, 128, 0, False),  # one chunk, a last tile of one row
+    (True, 32, 5000, 384, 1, True),  # an odd number of chunks: one per step
+    (True, 33, 5000, 384, 0, True),
+    (True, 64, 2 * 20488, 256, 2, False),  # more tiles than CUs: several items per block
+    (True, 5, 16384, 256, 0, False),  # two chunks per step
+    (True, 64, 96, 4096, 1, False),  # K split over the whole device
+    (False, 1, 33, 128, 0, False), (False, 32, 2 * 2500, 384, 2, False), (False, 33, 5000, 640, 1, False),
+    (False, 64, 40968, 256, 0, False), (False, 7, 4096, 512, 1, False), (False, 64, 96, 4096, 1, False)])
+def test_gemm_ring_edges(fp8, M, N, K, epi, mapped):
+    """The ring-staged form at the edges of its tiles, steps and items, same
+    bounds as the tests above (FP8 with the reference's +-480 codes)."""
+    if fp8:
+        test_gemm_fp8_mfma_within_tolerance(M, N, K, epi, mapped, True)
+    else:
+        test_gemm_mfma_within_tolerance(M, N, K, epi, True)
+
+
+@pytest.mark.parametrize("fp8,N,K", [(True, 5120, 2048), (True, 9000, 768), (False, 5120, 2048), (False, 9000, 640)])
+def test_gemm_ring_rows_do_not_depend_on_the_row_count(fp8, N, K):
+    """A row gives the same bits whether the call has 4, 32, 33 or 64 rows
+    (a verify and a correction of the same row round alike)."""
+    rng = np.random.default_rng(N + K)
+    x, xb = rand_bf16(rng, (64, K))
+    if fp8:
+        q, s = _fp8_weights(rng, N, K)
+        dw, ds = dev(q), dev(s)
+    else:
+        dw, ds = dev(rand_bf16(rng, (N, K), 0.05)[1]), None
+    dx = dev(xb)
+    rows = []
+    for M in (4, 32, 33, 64):
+        dy = out_buf(M * N * 2)
+        wsb = kern().hai_gemm_mfma_workspace_bytes(M, N)
+        dws = out_buf(max(wsb, 16))
+        if fp8:
+            hai.check(kern().hai_gemm_fp8_mfma(dy.ptr, N, dx.ptr, K, dw.ptr, ds.ptr, None, M, N, K,
+                                               hai.FP8_NO_SPECIAL_CODES, None, 0, dws.ptr, wsb, None), "fp8 mfma")
+        else:
+            hai.check(kern().hai_gemm_bf16_mfma(dy.ptr, N, dx.ptr, K, dw.ptr, M, N, K, 0, None, 0, dws.ptr, wsb,
+                                                None), "bf16 mfma")
+        rows.append(dy.download(np.uint16).reshape(M, N)[:4])
+    for r in rows[1:]:
+        assert np.array_equal(r, rows[0])
+
+
 @pytest.mark.parametrize("M,N,K,epi", [(32, 34816, 5120, 2), (32, 5120, 17408, 1), (64, 16480, 5120, 0)])
 def test_gemm_mfma_27b_shapes(M, N, K, epi):
     """The batched-verify GEMMs at their C4 (M = 8 sequences x 4 rows) and C5

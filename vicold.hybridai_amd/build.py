@@ -43,7 +43,8 @@ HIP_FLAGS = [
 CXX_FLAGS = ["-O2", "-fPIC", "-std=c++20", "-Wall", "-Wextra", "-Wno-unused-parameter",
              f"-I{INCLUDE}", f"-I{HOST}"]
 
-KERNEL_SOURCES = ["hai_runtime.hip", "hai_gemm.hip", "hai_gemm_fp8.hip", "hai_gemm_mfma.hip", "hai_norm.hip", "hai_attention.hip",
+KERNEL_SOURCES = ["hai_runtime.hip", "hai_gemm.hip", "hai_gemm_fp8.hip", "hai_gemm_mfma.hip", "hai_gemm_ring.hip",
+                  "hai_norm.hip", "hai_attention.hip",
                   "hai_deltanet.hip", "hai_deltanet_prefill.hip", "hai_argmax.hip"]
 
 

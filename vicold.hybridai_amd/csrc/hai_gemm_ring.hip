@@ -1,0 +1,490 @@
+// hai_gemm_ring.hip -- batched-verify linear layer, ring-staged form (see
+// hai_gemm_mfma.hip for the contract and the other forms).
+#include <atomic>
+#include <type_traits>
+
+#include "hai_common.h"
+#include "hai_device.h"
+#include "hai_gemm_common.h"
+#include "hai_gemm_ring.h"
+#include "hai_mfma.h"
+
+namespace {
+
+using namespace hai;
+
+// ---------------------------------------------------------------------------
+// Ring-staged batched GEMM (bf16 and FP8 weights, up to 64 rows, K a multiple
+// of 128).  A persistent block owns R weight rows (a multiple of 16, chosen so
+// that the tiles fill the CUs, see ring_plan) and walks its items (tile, range
+// of 128-k chunks) through two rings of LDS stages, weights [R] x 128 KC with
+// their scales (FP8) and activations [32 MT] x 128 KC:
+//   * two waves copy the weights and scales, SW - 1 stages ahead of the
+//     products, across item boundaries too, and the computing waves copy the
+//     activations (from L2) two stages ahead in their own in-order queue; each
+//     waits for its oldest stage with a counted s_waitcnt.  The copies are
+//     inline assembly, so that the compiler does not wait for them before its
+//     LDS reads;
+//   * NG x MT computing waves own 32 weight rows x 32 activation rows each:
+//     codes decoded exactly to bf16 in the B operand, a chunk (one 128-k scale
+//     block) summed by 8 MFMAs of 32 x 32 x 16, scaled in fp32;
+//   * one barrier per step of KC chunks: the step's stages have landed and
+//     those of the step before are free.
+// Rows sit in LDS with their 16-byte pieces permuted (piece p of row r at p ^
+// swizzle(r)) so that the rows of one operand read fall in distinct banks.
+// Rows past N and M repeat the last row (never stored); columns past R of the
+// last 32-row group read other LDS bytes (never stored either).
+// Bound by the copies: weights and activations share a CU's 27-32 B per ns
+// (about 64 KB in flight at the latency of HBM under load), so the activations,
+// re-read once per R rows, weigh as much per byte as the weights.  MI355X,
+// M = 64 FP8: gate|up 80 -> 50 us without a second pass, down 38 -> 30 us;
+// M = 32 bf16: gate|up 71 -> 56, down 38 -> 32 us.
+// ---------------------------------------------------------------------------
+constexpr int kRingCopiers = 2;   // waves that copy weights
+constexpr int kRingXStages = 3;   // activation stages
+constexpr int kRingLds = 160 * 1024;
+constexpr int kRingMaxStages = 12;
+
+// Weight stages that fit beside the activations, with the copies of all but
+// two of them in a wave's vmcnt range.
+int ring_stages(int R, int mt, bool fp8, int kc) {
+    const int ng = (R + 31) / 32;
+    const int w = R * kc * kRingK * (fp8 ? 1 : 2);
+    const int per = w / (1024 * kRingCopiers) + (fp8 ? (kc * ng + kRingCopiers - 1) / kRingCopiers : 0);
+    int n = (kRingLds - kRingXStages * 32 * mt * kc * kRingK * 2) / (w + (fp8 ? kc * ng * 256 : 0));
+    if (n > kRingMaxStages) n = kRingMaxStages;
+    while (n > 2 && (n - 2) * per > 63) --n;
+    return n;
+}
+
+// Chunks per step.  Two where one chunk is too little work between barriers:
+// up to 32 rows (one computing wave per 32 weight rows) and short tiles.
+int ring_kc(int R, int M, int K, bool fp8) { return M <= 32 && R <= (fp8 ? 96 : 64) && K % (2 * kRingK) == 0 ? 2 : 1; }
+
+template <int MT, int NG, bool FP8, int KC>
+struct RingShape {
+    static constexpr int EB = FP8 ? 1 : 2;
+    static constexpr int WROW = KC * kRingK * EB;         // bytes of a staged weight row
+    static constexpr int XROW = KC * kRingK * 2;          // bytes of a staged activation row
+    static constexpr int SB = FP8 ? KC * NG * 256 : 0;    // scale bytes of a weight stage
+    static constexpr int XB = 32 * MT * XROW;             // bytes of an activation stage
+    static constexpr int SX = kRingXStages;
+    static constexpr int WAVES = NG * MT + kRingCopiers;
+    static constexpr int SCALE_COPIES = FP8 ? (KC * NG + kRingCopiers - 1) / kRingCopiers : 0;  // per copying wave
+    static constexpr int XCOPIES = (XB / 1024 + NG * MT - 1) / (NG * MT);                  // per computing wave
+    __host__ __device__ static constexpr int w_stage(int R) { return R * WROW + SB; }
+    // 16-byte piece positions within a row
+    static __device__ __forceinline__ int w_swz(int r) { return WROW == 128 ? (r >> 1) & 7 : r & 15; }
+    static __device__ __forceinline__ int x_swz(int r) { return r & 15; }
+};
+
+// s_waitcnt vmcnt(n) for a run-time (wave-uniform) n.
+__device__ __forceinline__ void wait_vmcnt_n(int n) {
+    switch (n) {
+#define HAI_VM(v) case v: wait_vmcnt<v>(); break;
+#define HAI_VM8(v) HAI_VM(v) HAI_VM(v + 1) HAI_VM(v + 2) HAI_VM(v + 3) HAI_VM(v + 4) HAI_VM(v + 5) HAI_VM(v + 6) HAI_VM(v + 7)
+        HAI_VM8(0) HAI_VM8(8) HAI_VM8(16) HAI_VM8(24) HAI_VM8(32) HAI_VM8(40) HAI_VM8(48) HAI_VM8(56)
+#undef HAI_VM8
+#undef HAI_VM
+        default: wait_vmcnt<0>(); break;
+    }
+}
+// A wave-uniform pointer in scalar registers.
+__device__ __forceinline__ const void* uniform_ptr(const void* p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+    return reinterpret_cast<const void*>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+// One global -> LDS copy per lane of 16 (4) bytes at base + off, to lds + 16
+// (4) * lane (the M0 write needs one wait state); nt: non-temporal.
+__device__ __forceinline__ void ring_copy16(uint32_t off, const void* base, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds) : "memory");
+}
+__device__ __forceinline__ void ring_copy16_nt(uint32_t off, const void* base, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(off), "s"(base), "s"(lds) : "memory");
+}
+__device__ __forceinline__ void ring_copy4(uint32_t off, const void* base, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds) : "memory");
+}
+__device__ __forceinline__ u32x4 ring_read16(uint32_t lds) {
+    return *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)lds;
+}
+template <int MT, int NG, bool FP8, bool CHECK, int KC>
+__global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_kernel(RingArgs a, int SW) {
+    using SH = RingShape<MT, NG, FP8, KC>;
+    constexpr int SX = SH::SX;
+    extern __shared__ __align__(1024) uint8_t ring_lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = wave_index();
+    const int lc = lane & 31, lh = lane >> 5;
+    const int nck = a.K / (KC * kRingK);  // steps of KC chunks
+    const int R = a.R;
+    const int wstage = SH::w_stage(R);
+    const uint32_t lds0 = static_cast<uint32_t>(
+        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)ring_lds));
+    const uint32_t ldsx = lds0 + SW * wstage;  // the activation stages
+    // weights that the 256 MB cache behind the L2s cannot hold beside others are streamed past it (MI355X, gate|up
+    // FP8, 178 MB, M = 32: 47.7 -> 42.1 us with the norm; 16384 x 5120, 84 MB: 24.2 -> 24.8)
+    const bool nt = static_cast<int64_t>(a.N) * a.K * SH::EB > (int64_t{96} << 20);
+    const int items = a.tiles * a.splits;
+    auto chunk_lo = [&](int split) { return static_cast<int>(static_cast<int64_t>(split) * nck / a.splits); };
+    // total chunks of this block
+    int total = 0;
+    for (int it = blockIdx.x; it < items; it += gridDim.x)
+        total += chunk_lo(it / a.tiles + 1) - chunk_lo(it / a.tiles);
+
+    if (wave >= NG * MT) {  // ---- a copying wave: weights and scales ----
+        const int p = wave - NG * MT;
+        const int per = R * SH::WROW / (1024 * kRingCopiers) + SH::SCALE_COPIES;  // copies per chunk
+        constexpr int WL = 1024 / SH::WROW;  // weight rows per copy
+        const int wr = lane / (64 / WL), wpos = lane % (64 / WL);
+        // the chunk cursor: requests run ahead of the products
+        int item = blockIdx.x, c = 0, cend = 0, slot = 0;
+        uint32_t srow[SH::SCALE_COPIES > 0 ? SH::SCALE_COPIES : 1] = {};
+        const char* wbase = nullptr;
+        int last = 0;
+        auto open_item = [&]() {  // (item < items)
+            const int tile = item % a.tiles;
+            const int split = item / a.tiles;
+            c = chunk_lo(split);
+            cend = chunk_lo(split + 1);
+            const int64_t row0 = static_cast<int64_t>(tile) * R;
+            last = static_cast<int>(min(static_cast<int64_t>(R), a.N - row0)) - 1;
+            wbase = static_cast<const char*>(a.w) + row0 * a.K * SH::EB;
+            if constexpr (FP8) {
+                const int nkb = a.K / 128;
+#pragma unroll
+                for (int i = 0; i < SH::SCALE_COPIES; ++i) {
+                    const int g = min(p + kRingCopiers * i, KC * NG - 1);  // (row group g / KC, chunk g % KC)
+                    const int64_t n = min(row0 + 32 * (g / KC) + lc, static_cast<int64_t>(a.N) - 1);
+                    const int64_t nsb = ((a.N >> 1) + 127) / 128;
+                    const int64_t sr =
+                        a.scale_rows ? a.scale_rows[n] : (a.paired ? (n & 1) * nsb + (n >> 1) / 128 : n / 128);
+                    srow[i] = static_cast<uint32_t>((sr * nkb + g % KC) * 4);
+                }
+            }
+        };
+        // this wave's copies of a stage are i = p + 2 t; the piece permutation of a lane's row repeats every four,
+        // so a whole tile needs four lane offsets and a scalar base per copy
+        constexpr int PH = 4;
+        const int ncopy = R / (WL * kRingCopiers);
+        const uint32_t wpitch = static_cast<uint32_t>(a.K) * SH::EB;
+        uint32_t woff[PH];
+#pragma unroll
+        for (int u = 0; u < PH; ++u)
+            woff[u] = wr * wpitch + ((wpos ^ SH::w_swz((p + kRingCopiers * u) * WL + wr)) << 4);
+        auto copy_w = [&](auto stream, const void* wb, uint32_t dst) {
+            constexpr bool NT = decltype(stream)::value;
+            if (last == R - 1) {
+                const char* base = static_cast<const char*>(wb) + static_cast<int64_t>(p * WL) * wpitch;
+                const int64_t step = static_cast<int64_t>(kRingCopiers * WL) * wpitch;
+                dst += p * 1024;
+                for (int t = 0; t < ncopy; t += PH) {
+#pragma unroll
+                    for (int u = 0; u < PH; ++u) {
+                        if (t + u >= ncopy) break;
+                        if constexpr (NT) ring_copy16_nt(woff[u], base, dst);
+                        else ring_copy16(woff[u], base, dst);
+                        base += step;
+                        dst += kRingCopiers * 1024;
+                    }
+                }
+            } else {  // rows past N: the last one
+                for (int t = 0; t < ncopy; ++t) {
+                    const int i = p + kRingCopiers * t;
+                    const int r = i * WL + wr;
+                    const uint32_t off = static_cast<uint32_t>(min(r, last)) * wpitch + ((wpos ^ SH::w_swz(r)) << 4);
+                    if constexpr (NT) ring_copy16_nt(off, wb, dst + i * 1024);
+                    else ring_copy16(off, wb, dst + i * 1024);
+                }
+            }
+        };
+        auto request = [&]() {  // the cursor's chunk into the next slot
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + slot * wstage);
+            const void* wb = uniform_ptr(wbase + static_cast<int64_t>(c) * SH::WROW);
+            if (nt) copy_w(std::true_type{}, wb, dst);
+            else copy_w(std::false_type{}, wb, dst);
+            if constexpr (FP8) {
+#pragma unroll
+                for (int i = 0; i < SH::SCALE_COPIES; ++i)
+                    ring_copy4(srow[i] + c * (4 * KC), a.scales,
+                               dst + R * SH::WROW + min(p + kRingCopiers * i, KC * NG - 1) * 256);
+            }
+            slot = slot + 1 == SW ? 0 : slot + 1;
+            if (++c == cend) {
+                item += gridDim.x;
+                if (item < items) open_item();
+            }
+        };
+        open_item();
+        int asked = 0;
+        for (; asked < SW - 1 && asked < total; ++asked) request();
+        for (int i = 0; i < total; ++i) {
+            // chunk i has landed: at most the later chunks' requests are outstanding
+            if (i + SW - 2 < total) wait_vmcnt_n((SW - 2) * per);
+            else wait_vmcnt<0>();
+            lds_barrier();
+            if (asked < total) {
+                request();
+                ++asked;
+            }
+        }
+        return;
+    }
+
+    // ---- a computing wave: weight rows 32 ng .. + 31, activation rows 32 mg .. + 31 ----
+    const int ng = wave % NG, mg = wave / NG;
+    const int wrow = 32 * ng + lc, xrow = 32 * mg + lc;
+    const uint32_t w0 = lds0 + wrow * SH::WROW, x0 = ldsx + xrow * SH::XROW;
+    const int wsw = SH::w_swz(wrow), xsw = SH::x_swz(xrow);
+    // its share of the activation copies (the last ones of an uneven split repeat the last 1 KB)
+    constexpr int XLANES = SH::XROW / 16;  // lanes per row
+    uint32_t xoff[SH::XCOPIES], xdst[SH::XCOPIES];
+#pragma unroll
+    for (int j = 0; j < SH::XCOPIES; ++j) {
+        const int i = min(wave + NG * MT * j, SH::XB / 1024 - 1);
+        const int r = i * (64 / XLANES) + lane / XLANES;
+        xoff[j] = static_cast<uint32_t>(min(r, a.M - 1)) * static_cast<uint32_t>(a.ldx * 2) +
+                  (((lane % XLANES) ^ SH::x_swz(r)) << 4);
+        xdst[j] = __builtin_amdgcn_readfirstlane(ldsx + i * 1024);
+    }
+    int xitem = blockIdx.x, xc = chunk_lo(xitem / a.tiles), xend = chunk_lo(xitem / a.tiles + 1), xslot = 0, xasked = 0;
+    auto request_x = [&]() {
+        const void* xb = uniform_ptr(reinterpret_cast<const char*>(a.x) + static_cast<int64_t>(xc) * SH::XROW);
+#pragma unroll
+        for (int j = 0; j < SH::XCOPIES; ++j)
+            ring_copy16(xoff[j], xb, __builtin_amdgcn_readfirstlane(xdst[j] + xslot * SH::XB));
+        xslot = xslot + 1 == SX ? 0 : xslot + 1;
+        ++xasked;
+        if (++xc == xend) {
+            xitem += gridDim.x;
+            if (xitem < items) {
+                xc = chunk_lo(xitem / a.tiles);
+                xend = chunk_lo(xitem / a.tiles + 1);
+            }
+        }
+    };
+    while (xasked < SX - 1 && xasked < total) request_x();
+    int done = 0, slot = 0, xs = 0;
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        const int tile = item % a.tiles;
+        const int split = item / a.tiles;
+        const int cend = chunk_lo(split + 1);
+        f32x16 tot;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) tot[i] = 0.0f;
+        for (int c = chunk_lo(split); c < cend; ++c) {
+            // this wave's copies of the chunk have landed, then everyone's
+            if (done + SX - 2 < total) wait_vmcnt<(SX - 2) * SH::XCOPIES>();
+            else wait_vmcnt<0>();
+            lds_barrier();
+            if (xasked < total) request_x();
+            ++done;
+            const uint32_t so = slot * wstage, xo = xs * SH::XB;
+            slot = slot + 1 == SW ? 0 : slot + 1;
+            xs = xs + 1 == SX ? 0 : xs + 1;
+            if constexpr (FP8) {
+                // step 2 j + e of chunk q: k = 32 j + 16 lh + 8 e + [0, 8); the next pair's activations are read
+                // while a pair's codes are decoded and multiplied
+                auto x_at = [&](int q, int j) {
+                    return ring_read16(x0 + xo + (((16 * q + 4 * (j >> 1) + 2 * lh + (j & 1)) ^ xsw) << 4));
+                };
+                u32x4 wq[KC][4], xa[2][KC][2];
+                float sc[KC];
+#pragma unroll
+                for (int q = 0; q < KC; ++q) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        wq[q][j] = ring_read16(w0 + so + (((8 * q + 2 * j + lh) ^ wsw) << 4));
+                    xa[0][q][0] = x_at(q, 0);
+                    xa[0][q][1] = x_at(q, 1);
+                    sc[q] = *(const __attribute__((address_space(3))) float*)(uintptr_t)(
+                        lds0 + so + R * SH::WROW + (ng * KC + q) * 256 + lc * 4);
+                }
+                // (one chain of products per chunk in every form, so that a row's sums do not depend on how many
+                // rows the call has)
+                f32x16 acc[KC];
+#pragma unroll
+                for (int q = 0; q < KC; ++q)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[q][i] = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    u32x4 d[KC][2];
+#pragma unroll
+                    for (int q = 0; q < KC; ++q) {
+                        if (j < 3) {
+                            xa[(j + 1) & 1][q][0] = x_at(q, 2 * j + 2);
+                            xa[(j + 1) & 1][q][1] = x_at(q, 2 * j + 3);
+                        }
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            uint32_t lo, hi;
+                            if constexpr (CHECK) {
+                                e4m3x4_to_bf16<true>(wq[q][j][e], lo, hi);
+                            } else {
+                                lo = e4m3x2_to_bf16(wq[q][j][e], false);
+                                hi = e4m3x2_to_bf16(wq[q][j][e], true);
+                            }
+                            d[q][e >> 1][2 * (e & 1)] = lo;
+                            d[q][e >> 1][2 * (e & 1) + 1] = hi;
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int q = 0; q < KC; ++q) acc[q] = mfma32(xa[j & 1][q][e], d[q][e], acc[q]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int q = 0; q < KC; ++q)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) tot[i] = fma_(sc[q], acc[q][i], tot[i]);
+            } else {
+                u32x4 wb[8], xa[8];
+#pragma unroll
+                for (int q = 0; q < KC; ++q) {
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        wb[t] = ring_read16(w0 + so + (((16 * q + 2 * t + lh) ^ wsw) << 4));
+                        xa[t] = ring_read16(x0 + xo + (((16 * q + 2 * t + lh) ^ xsw) << 4));
+                    }
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) tot = mfma32(xa[t], wb[t], tot);
+                }
+            }
+        }
+        // result: lane = weight row (column n), element i = activation row 8 (i / 4) + 4 lh + i % 4
+        const int64_t n = static_cast<int64_t>(tile) * R + wrow;
+        const bool col = wrow < R && n < a.N;
+        const int m0 = 32 * mg + 4 * lh;
+        if (a.splits > 1) {
+            if (col) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int m = m0 + 8 * (i >> 2) + (i & 3);
+                    if (m < a.M) a.part[(static_cast<int64_t>(split) * a.M + m) * a.N + n] = tot[i];
+                }
+            }
+        } else if (a.epi == HAI_EPI_SILU_MUL) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int m = m0 + 8 * (i >> 2) + (i & 3);
+                const float g = bfr(tot[i]);
+                const float u = quad_xor1(g);
+                if ((lc & 1) == 0 && col && m < a.M)
+                    a.y[static_cast<int64_t>(m) * a.ldy + n / 2] = f2bf(fast_silu(g) * u);
+            }
+        } else if (col) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int m = m0 + 8 * (i >> 2) + (i & 3);
+                if (m >= a.M) continue;
+                float o = bfr(tot[i]);
+                if (a.epi == HAI_EPI_RESIDUAL) o = bf2f(a.res[static_cast<int64_t>(m) * a.ldres + n]) + o;
+                a.y[static_cast<int64_t>(m) * a.ldy + n] = f2bf(o);
+            }
+        }
+    }
+}
+
+template <int MT, int NG, bool FP8, bool CHECK, int KC = 1>
+int launch_ring_as(const RingArgs& r, int cus, hipStream_t s) {
+    using SH = RingShape<MT, NG, FP8, KC>;
+    static std::atomic<uint8_t> allowed[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return invalid("gemm_mfma: device");
+    auto* kern = gemm_ring_mfma_kernel<MT, NG, FP8, CHECK, KC>;
+    if (!allowed[dev].load(std::memory_order_acquire)) {
+        const int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds),
+                                 "hipFuncSetAttribute");
+        if (rc != HAI_OK) return rc;
+        allowed[dev].store(1, std::memory_order_release);
+    }
+    const int sw = ring_stages(r.R, MT, FP8, KC);
+    const size_t shmem = static_cast<size_t>(sw) * SH::w_stage(r.R) + SH::SX * SH::XB;
+    const int64_t items = static_cast<int64_t>(r.tiles) * r.splits;
+    const unsigned grid = static_cast<unsigned>(items < cus ? items : cus);
+    kern<<<dim3(grid), dim3(64 * SH::WAVES), shmem, s>>>(r, sw);
+    return launched("gemm_ring_mfma_kernel");
+}
+template <int MT, bool FP8, bool CHECK>
+int launch_ring_ng(const RingArgs& r, int cus, hipStream_t s) {
+    if constexpr (MT == 1) {
+        if (ring_kc(r.R, r.M, r.K, FP8) == 2) {
+            if (r.R <= 32) return launch_ring_as<MT, 1, FP8, CHECK, 2>(r, cus, s);
+            if (r.R <= 64) return launch_ring_as<MT, 2, FP8, CHECK, 2>(r, cus, s);
+            if constexpr (FP8) return launch_ring_as<MT, 3, FP8, CHECK, 2>(r, cus, s);
+        }
+    }
+    switch ((r.R + 31) / 32) {
+        case 1: return launch_ring_as<MT, 1, FP8, CHECK>(r, cus, s);
+        case 2: return launch_ring_as<MT, 2, FP8, CHECK>(r, cus, s);
+        case 3: return launch_ring_as<MT, 3, FP8, CHECK>(r, cus, s);
+        case 4: return launch_ring_as<MT, 4, FP8, CHECK>(r, cus, s);
+        default: return launch_ring_as<MT, 5, FP8, CHECK>(r, cus, s);
+    }
+}
+
+}  // namespace
+
+namespace hai {
+
+// The plan whose busiest CU copies the fewest bytes: the copies are what
+// bounds the kernel, weights (HBM) and activations (L2) alike, at 27-32 B per
+// ns and CU however many stages are in flight (MI355X, M = 64 FP8: gate|up,
+// 242 tiles of 144 rows, W alone 34 us, X alone 17, both 48).  A split adds its
+// partial planes and a second pass (about 9 us with its launch: 16384 x 5120 at
+// M = 64, 256 tiles of 64 33.5 us, 128 tiles of 128 in two splits 36.2).
+// The splits follow N, K and the weight format alone (priced for 64 rows), so
+// that a row's sums are the same whatever the number of rows: a verify and a
+// correction of the same row round alike.
+void ring_plan(RingArgs& r, int max_splits, bool fixed, int cus) {
+    const bool fp8 = r.scales != nullptr;
+    const int eb = fp8 ? 1 : 2;
+    const int64_t nck = r.K / kRingK;
+    // the best tile height for `splits` splits of M rows, and its cost
+    auto best_tile = [&](int M, int splits, double& cost) {
+        const int mt = M <= 32 ? 1 : 2;
+        int best = 0;
+        for (int R = 32; R <= 160; R += 16) {
+            if (ring_stages(R, mt, fp8, ring_kc(R, M, r.K, fp8)) < 3) break;
+            const int64_t tiles = (static_cast<int64_t>(r.N) + R - 1) / R;
+            const int64_t rounds = (tiles * splits + cus - 1) / cus;
+            const double c = static_cast<double>(rounds) * static_cast<double>((nck + splits - 1) / splits) *
+                             (R * kRingK * eb + mt * 32 * kRingK * 2);
+            if (best == 0 || c < cost) {
+                best = R;
+                cost = c;
+            }
+        }
+        return best;
+    };
+    r.splits = max_splits;
+    double cost = 0.0;
+    for (int splits = 1; splits <= max_splits && !fixed; ++splits) {
+        double c = 0.0;
+        best_tile(kRingMaxRows, splits, c);
+        if (splits > 1) c += 270e3 + 8.0 * splits * kRingMaxRows * r.N / cus;
+        if (splits == 1 || c < cost) {
+            r.splits = splits;
+            cost = c;
+        }
+    }
+    r.R = best_tile(r.M, r.splits, cost);
+    r.tiles = (r.N + r.R - 1) / r.R;
+}
+
+int launch_ring(const RingArgs& r, bool check, int cus, hipStream_t s) {
+    if (r.M <= 32)
+        return r.scales == nullptr ? launch_ring_ng<1, false, false>(r, cus, s)
+               : check             ? launch_ring_ng<1, true, true>(r, cus, s)
+                                   : launch_ring_ng<1, true, false>(r, cus, s);
+    return r.scales == nullptr ? launch_ring_ng<2, false, false>(r, cus, s)
+           : check             ? launch_ring_ng<2, true, true>(r, cus, s)
+                               : launch_ring_ng<2, true, false>(r, cus, s);
+}
+
+}  // namespace hai
