@@ -538,12 +538,11 @@ __global__ __launch_bounds__(256) void gemm_fp8_mfma_kernel(uint16_t* __restrict
 constexpr int kRtChunk = 256;  // k per chunk of the copy-staged kernel (two 128-k halves)
 
 // ---------------------------------------------------------------------------
-// Copy-staged variant for FP8 weights on the wide layers at 17-64 rows: the
-// register-operand kernel's tile, roles and arithmetic (a wave owns 32
-// weight rows and one 128-k half of every 256-k chunk, codes decoded
-// exactly to bf16 in its B operands, scale blocks applied in fp32), with
-// every operand staged by global -> LDS copies instead of registers, so
-// that the weight bytes in flight are bounded by LDS rather than by VGPRs:
+// Copy-staged variant for FP8 weights on wide layers at 17-64 rows: a block
+// owns 64 weight rows (a wave 32 of them and one 128-k half of every 256-k
+// chunk, codes decoded exactly to bf16 in its B operands, scale blocks applied
+// in fp32), every operand staged by global -> LDS copies, so that the weight
+// bytes in flight are bounded by LDS rather than by VGPRs:
 //   * three weight stages (64 rows x 256 codes, 16 KB, and behind them the
 //     chunk's scales, one 4-byte copy per lane and n-tile) and three
 //     activation stages (16 MT rows x 256 bf16); the weights, scales and
@@ -556,8 +555,7 @@ constexpr int kRtChunk = 256;  // k per chunk of the copy-staged kernel (two 128
 //   * a wave copies and reads only its own weight region (32 rows x 128
 //     bytes, row r's 16-byte piece p at slot p ^ (r & 7)); the activation
 //     stages are filled by all four waves (row r's piece p at slot
-//     p ^ (r & 15), as the register-operand kernel stores them) and read by
-//     all behind a barrier.
+//     p ^ (r & 15)) and read by all behind a barrier.
 // Weight rows past N and activation rows past M are read from the last row
 // (their results are never stored); chunks past K from the last chunk
 // (never used).
@@ -869,7 +867,12 @@ int device_cus();
 // 64 80.5 / 55.6, M = 32 55 / 45, M = 4 44.6 / 44.6; bf16 M = 32 75 / 61, M = 64
 // 95 / 67; 16384 x 5120 FP8 35 / 32, bf16 M = 64 47 / 40; 5120 x 8192 FP8 27.8 /
 // 25.1; 8192 x 1024 17.5 / 12.5.  (Closest: 16384 x 5120 FP8 at 17-32 rows, 23.6
-// / 24.1.)  K not a multiple of 128 and 65-128 rows keep the kernels here.
+// / 24.1.)  An odd number of chunks leaves one per step, which one computing
+// wave per block does not hide up to 32 rows, while from 33 rows on the ring
+// is ahead: LDS-staged / ring, 5568 x 2944 FP8 M = 5 16.6 / 18.6, M = 28 16.1 /
+// 18.4, M = 64 20.6 / 19.0 (bf16 21.7 / 19.0), 8192 x 4992 FP8 M = 32 20.8 /
+// 18.6.  The line does not follow M, so that a row rounds alike in calls of
+// any size.  K not a multiple of 128 and 65-128 rows keep the kernels here.
 bool ring_shape(int64_t M, int64_t K) { return K % kRingK == 0 && M <= kRingMaxRows; }
 
 // LDS above the 64 KB default needs the attribute, once per kernel instance.
