@@ -622,6 +622,29 @@ def test_gqa_verify_mfma_flash(B, T, nq, nkv, D, lens):
     test_gqa_verify_mfma(B, T, nq, nkv, D, lens)
 
 
+@pytest.mark.parametrize("B,T,nq,nkv,D", [(2, 513, 24, 8, 64), (3, 345, 12, 4, 128), (2, 257, 24, 4, 256),
+                                          (6, 258, 24, 4, 256)])
+def test_gqa_flash_weights_sum_to_one(B, T, nq, nkv, D):
+    """The flash form normalises by the sum of the weights as it multiplies
+    them with V (rounded to bf16), so they sum to one to fp32 accuracy: when
+    every key of a head holds the same bf16 value the output is that value."""
+    rng = np.random.default_rng(D + T)
+    cap = T + 700
+    v1, v1b = rand_bf16(rng, (nkv, D))
+    q, qb = rand_bf16(rng, (B * T, nq, D), 2.0)
+    _, kb = rand_bf16(rng, (B, cap, nkv, D))
+    vb = np.ascontiguousarray(np.broadcast_to(v1b.reshape(nkv, D), (B, cap, nkv, D)))
+    dq, dk, dv = dev(qb), dev(kb), dev(vb)
+    dl = dev(rng.integers(0, 690, B).astype(np.int32))
+    scratch = out_buf(kern().hai_gqa_mfma_scratch_bytes(B, T, nq, D, cap))
+    dout = out_buf(B * T * nq * D * 2)
+    hai.check(kern().hai_gqa_verify_mfma_bf16(dout.ptr, dq.ptr, None, dk.ptr, dv.ptr, cap, scratch.ptr, B, T, nq,
+                                              nkv, D, dl.ptr, T, cap, None), "gqa mfma")
+    got = dout.download(np.uint16).reshape(B * T, nq, D)
+    bad = got != np.repeat(v1b.reshape(nkv, D), nq // nkv, 0)[None]
+    assert not bad.any(), int(bad.sum())
+
+
 # ----------------------------------------------------------------- deltanet
 def _deltanet_case(rng, B, nk, nv, dk, dv, Kc=4):
     kw, vw = nk * dk, nv * dv

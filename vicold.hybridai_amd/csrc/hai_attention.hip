@@ -505,6 +505,7 @@ int launch(uint16_t* out, const uint16_t* q, const uint16_t* gate, const uint16_
 // ---------------------------------------------------------------------------
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -1168,9 +1169,14 @@ __global__ __launch_bounds__(64 * W) void gqa_fa_kernel(uint16_t* __restrict__ o
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const float p = __builtin_amdgcn_exp2f(fma_(st[i], scale_log2, sub));
-                ps[i & 1] += p;
                 pb[i >> 3][i & 7] = static_cast<__bf16>(p);
             }
+            // the normaliser sums the weights as P V takes them, rounded: a rounding then moves the output by
+            // delta (v - O) and not by delta v
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                ps[i & 1] = __builtin_amdgcn_fdot2_f32_bf16(
+                    bf16x2{pb[i >> 2][2 * (i & 3)], pb[i >> 2][2 * (i & 3) + 1]}, bf16x2{1.0f, 1.0f}, ps[i & 1], false);
             l += ps[0] + ps[1];
             // ---- O^T += V^T P^T: k step s covers keys 16 s + (4 lh + q % 4 + 8 (q / 4)), q the k slot ----
 #pragma unroll
