@@ -645,6 +645,39 @@ def test_gqa_flash_weights_sum_to_one(B, T, nq, nkv, D):
     assert not bad.any(), int(bad.sum())
 
 
+@pytest.mark.parametrize("B,T,nq,nkv,D", [(2, 513, 24, 8, 64), (3, 345, 12, 4, 128), (2, 257, 24, 4, 256)])
+def test_gqa_flash_gate_every_bf16(B, T, nq, nkv, D):
+    """The flash form's epilogue over every bf16 gate.  Zero queries weigh all
+    keys alike (p = 1) and every key of a head holds the same value v, so the
+    output is v * sigmoid(gate) rounded to bf16: half a bf16 unit from float64,
+    and 2^-21 of it for the fp32 quotient, sigmoid and product, down to where
+    the canonical sigmoid's e^-gate overflows (gates below -88.72)."""
+    rng = np.random.default_rng(D)
+    n = B * T * nq * D
+    gb = np.resize(np.arange(65536, dtype=np.uint16), n)
+    g = hai.bf16_to_f32(gb).reshape(B, T, nq, D)
+    cap = T + 3
+    v1 = rng.integers(1, 8, (nkv, D)).astype(np.float32) * rng.choice([-1.0, 1.0], (nkv, D)).astype(np.float32)
+    v = np.broadcast_to(v1, (B, cap, nkv, D))
+    _, kb = rand_bf16(rng, (B, cap, nkv, D))
+    dq, dg, dk, dv = out_buf(n * 2), dev(gb), dev(kb), dev(hai.bf16_bits(np.ascontiguousarray(v)))
+    dl = dev(np.zeros(B, np.int32))
+    scratch = out_buf(kern().hai_gqa_mfma_scratch_bytes(B, T, nq, D, cap))
+    dout = out_buf(n * 2)
+    hai.check(kern().hai_gqa_verify_mfma_bf16(dout.ptr, dq.ptr, dg.ptr, dk.ptr, dv.ptr, cap, scratch.ptr, B, T, nq,
+                                              nkv, D, dl.ptr, T, cap, None), "gqa mfma")
+    got = dout.download(np.uint16)
+    g = g.reshape(-1).astype(np.float64)
+    with np.errstate(all="ignore"):
+        sig = np.where(g < -88.72284, 0.0, 1.0 / (1.0 + np.exp(-g)))
+    want = (np.repeat(v1, nq // nkv, 0)[None, None] * sig.reshape(B, T, nq, D)).reshape(-1)
+    got = hai.bf16_to_f32(got).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(g))
+    unit = 2.0 ** (np.maximum(np.floor(np.log2(np.maximum(np.abs(want), 1e-300))), -126) - 7)
+    bad = np.abs(got - want) > 0.5 * unit + 2.0 ** -21 * np.abs(want)
+    assert not bad.any(), (int(bad.sum()), g[bad][:8], got[bad][:8], want[bad][:8])
+
+
 # ----------------------------------------------------------------- deltanet
 def _deltanet_case(rng, B, nk, nv, dk, dv, Kc=4):
     kw, vw = nk * dk, nv * dv

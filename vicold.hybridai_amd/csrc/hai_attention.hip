@@ -1009,11 +1009,6 @@ __device__ __forceinline__ u32x4 fa_read16(uint32_t lds) {
     return *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)lds;
 }
 
-// 1 / (1 + e^-x) by the hardware exp2 and reciprocal (tolerance mode).
-__device__ __forceinline__ float fast_sigmoid(float x) {
-    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-}
-
 template <int D, int W>
 __global__ __launch_bounds__(64 * W) void gqa_fa_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
                                                         const uint16_t* __restrict__ gate, const uint16_t* kc,
@@ -1197,8 +1192,8 @@ __global__ __launch_bounds__(64 * W) void gqa_fa_kernel(uint16_t* __restrict__ o
     }
 
     // ---- O / l * sigmoid(gate), rounded: lane holds dims 32 dt + 8 (i / 4) + 4 lh + i % 4.  One reciprocal
-    // per query and the hardware exp2 / reciprocal (fp32, 1 ulp) for the gate: D / 2 IEEE divisions and
-    // canonical exps per lane were a third of the kernel's time at 1024 x 1024 ----
+    // per query and hw_sigmoid: D / 2 IEEE divisions and canonical exps per lane take 20 us a block (MI355X, 1 x
+    // 1024 rows over 1024 keys with the norms: 69.8 / 90.3) ----
     if (qi >= nqry) return;
     l += __shfl_xor(l, 32);
     const float inv = 1.0f / l;
@@ -1213,10 +1208,10 @@ __global__ __launch_bounds__(64 * W) void gqa_fa_kernel(uint16_t* __restrict__ o
             for (int e = 0; e < 4; ++e) v[e] = o[dt][4 * g4 + e] * inv;
             if (gate != nullptr) {
                 const uint2 gv = *reinterpret_cast<const uint2*>(gate + row * D + d);
-                v[0] *= fast_sigmoid(lo_bf(gv.x));
-                v[1] *= fast_sigmoid(hi_bf(gv.x));
-                v[2] *= fast_sigmoid(lo_bf(gv.y));
-                v[3] *= fast_sigmoid(hi_bf(gv.y));
+                v[0] *= hw_sigmoid(lo_bf(gv.x));
+                v[1] *= hw_sigmoid(hi_bf(gv.x));
+                v[2] *= hw_sigmoid(lo_bf(gv.y));
+                v[3] *= hw_sigmoid(hi_bf(gv.y));
             }
             *reinterpret_cast<uint2*>(out + row * D + d) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
         }
