@@ -950,6 +950,53 @@ def test_deltanet_prefill_forms(nk, nv, dk, T, Kc):
     test_deltanet_prefill_against_oracle(nk, nv, dk, T, Kc)
 
 
+@pytest.mark.parametrize("dk", [128, 64])
+def test_deltanet_prefill_chunk_values_keep_fp32(dk):
+    """U = (I + L)^-1 diag(beta) V, the chunk's values that the state pass
+    subtracts W^ S from, is an fp32 quantity.  With keys of disjoint support
+    and no decay L is zero and U = beta v: it may differ from float64 by the
+    sigmoid's fp32 roundings (hardware exp2 and reciprocal, |b| < 4: below 8
+    units of 2^-23), where a pair of bf16 for the factor would show 2^-18."""
+    rng = np.random.default_rng(dk)
+    T, nk, nv, dv, Kc, ring, nslots = 32, 2, 6, dk, 1, 32, 40
+    kw, vw = nk * dk, nv * dv
+    C = 2 * kw + vw
+    x = rng.uniform(-3.0, 3.0, (T, C + vw + 2 * nv)).astype(np.float32)
+    x = hai.bf16_to_f32(hai.bf16_bits(x))
+    per = dk // T
+    for h in range(nk):
+        for t in range(T):
+            row = np.zeros(dk, np.float32)
+            row[t * per:(t + 1) * per] = 1.0
+            x[t, kw + h * dk:kw + (h + 1) * dk] = row
+    pb = hai.bf16_bits(x)
+    ones, zeros = np.ones((C, Kc), np.float32), np.zeros(nv, np.float32)
+    lens = np.zeros(1, np.int32)
+    dp, dcw, dal, ddt = dev(pb), dev(hai.bf16_bits(ones)), dev(hai.bf16_bits(zeros)), dev(hai.bf16_bits(zeros - 30.0))
+    dnw, dlen = dev(hai.bf16_bits(np.ones(dv, np.float32))), dev(lens)
+    dring, dstate = out_buf(ring * C * 2), out_buf(nslots * nv * dv * dk * 4)
+    dout = out_buf(T * vw * 2)
+    wsb = kern().hai_deltanet_prefill_workspace_bytes(1, T, nv, dv)
+    dws = out_buf(wsb)
+    hai.check(kern().hai_deltanet_prefill_bf16(dout.ptr, vw, dp.ptr, x.shape[1], 0, C, C + vw, C + vw + nv, dcw.ptr,
+                                               dring.ptr, ring, dstate.ptr, nslots, dal.ptr, ddt.ptr, dnw.ptr,
+                                               dlen.ptr, 0, 1, T, nk, nv, dk, dv, Kc, 1e-6, dws.ptr, wsb, None),
+              "deltanet_prefill")
+    # the workspace: the unrounded outputs, then one record per head whose first T x dv floats are U
+    ws = dws.download(np.float32)[T * vw:].reshape(nv, -1)
+    U = ws[:, :T * dv].reshape(nv, T, dv)
+    xv = x[:, 2 * kw:C].astype(np.float64).reshape(T, nv, dv)
+    v = xv / (1.0 + np.exp(-xv))
+    tie = np.abs(np.frexp(v)[0] * 256.0 % 1.0 - 0.5)  # distance from a bf16 rounding tie
+    v = hai.bf16_to_f32(hai.bf16_bits(v.astype(np.float32))).astype(np.float64)
+    beta = 1.0 / (1.0 + np.exp(-x[:, C + vw + nv:].astype(np.float64)))
+    for h in range(nv):
+        want = beta[:, h, None] * v[:, h]
+        ok = (tie[:, h] > 1e-3) & (want != 0.0)
+        rel = np.abs(U[h] - want)[ok] / np.abs(want)[ok]
+        assert rel.max() <= 2.0 ** -20, (h, float(rel.max()))
+
+
 @pytest.mark.parametrize("B,nk,nv,dk,T,Kc,ab", [(3, 2, 6, 64, 40, 4, False), (2, 16, 48, 128, 33, 4, True),
                                                 (1, 4, 4, 64, 100, 3, False)])
 def test_deltanet_prompt_chunk_equals_16_token_launches(B, nk, nv, dk, T, Kc, ab):

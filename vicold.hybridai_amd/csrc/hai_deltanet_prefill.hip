@@ -95,6 +95,17 @@ __device__ __forceinline__ void dn_split8(const float (&x)[8], u32x4& hi, u32x4&
         lo[q] = f2bf2(x[2 * q] - lo_bf(hp), x[2 * q + 1] - hi_bf(hp));
     }
 }
+// x as three bf16 (largest first): the fp32 value whole
+__device__ __forceinline__ void dn_split8x3(const float (&x)[8], u32x4 (&p)[3]) {
+    float r[8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        p[0][q] = f2bf2(x[2 * q], x[2 * q + 1]);
+        r[2 * q] = x[2 * q] - lo_bf(p[0][q]);
+        r[2 * q + 1] = x[2 * q + 1] - hi_bf(p[0][q]);
+    }
+    dn_split8(r, p[1], p[2]);
+}
 // elements off .. off + 7 of an accumulator tile, split the same way
 __device__ __forceinline__ void dn_split8(const dn_f32x16& x, int off, u32x4& hi, u32x4& lo) {
 #pragma unroll
@@ -118,7 +129,10 @@ __device__ __forceinline__ dn_f32x16 dn_mfma(u32x4 a, u32x4 b, dn_f32x16 c) {
 // from the 32 x 32 inverse T = (I + L)^-1, found by forward substitution (one
 // wave, lane = column), as
 //   U = (T diag(beta)) V,   W^ = (T diag(beta e^g |k|^-1)) K
-// with T's factor split into a bf16 pair.  Each product is oriented so that
+// with T's factor split into three bf16 (all 24 bits: K and V are bf16, so the
+// products are those of fp32 factors; a pair leaves 2^-18 in U.  MI355X, the
+// whole call, pair / three: 1000 tokens of 48 heads 117.1 / 117.4 us, 32 x 512
+// 1067 / 1076).  Each product is oriented so that
 // its result tile is the operand table the next pass wants: P from K Q^T and
 // W^ from K^T T^T (lane = token, elements = tokens / keys in op_slot order).
 // Columns of K and V come out of their rows through the transposing LDS reads.
@@ -405,14 +419,14 @@ __global__ __launch_bounds__(256) void deltanet_chunk_prep_kernel(PrefillArgs A)
             }
 #pragma unroll
             for (int q = 0; q < 8; ++q) t8[q] *= f[q];
-            u32x4 th, tl;
-            dn_split8(t8, th, tl);
+            u32x4 t3[3];
+            dn_split8x3(t8, t3);
             const int r = 16 * st + 4 * lh + (li >> 2), cc = col0 + (lane & 16) + 4 * (li & 3);
             const uint16_t* at = isv ? &vs[r][cc] : &ks[r][cc];
             const uint2 a = dn_read_tr(at), b2 = dn_read_tr(at + 8 * (isv ? VP : QP));
             const u32x4 xb = u32x4{a.x, a.y, b2.x, b2.y};
-            R = isv ? dn_mfma(tl, xb, R) : dn_mfma(xb, tl, R);
-            R = isv ? dn_mfma(th, xb, R) : dn_mfma(xb, th, R);
+#pragma unroll
+            for (int e = 2; e >= 0; --e) R = isv ? dn_mfma(t3[e], xb, R) : dn_mfma(xb, t3[e], R);
         }
         if (isv) {  // row = token, column = value column
 #pragma unroll
