@@ -997,6 +997,36 @@ def test_deltanet_prefill_chunk_values_keep_fp32(dk):
         assert rel.max() <= 2.0 ** -20, (h, float(rel.max()))
 
 
+def test_deltanet_prefill_norm_forms_agree():
+    """The gated RMSNorm's 16-byte form and its two-byte form (output rows not
+    a multiple of 16 bytes apart) give the same bits, over gates out to where
+    sigmoid leaves the normal fp32 numbers."""
+    rng = np.random.default_rng(77)
+    B, T, nk, nv, dk, Kc, ring, nslots = 2, 70, 2, 6, 128, 4, 96, 80
+    dv = dk
+    vw, width = nv * dv, 2 * nk * dk + 2 * nv * dv + 16
+    c = _deltanet_case(rng, B, nk, nv, dk, dv, Kc)
+    C = c["C"]
+    proj, _ = rand_bf16(rng, (B * T, width))
+    proj[:, C:C + vw] *= 30.0
+    pb = hai.bf16_bits(proj)
+    outs = []
+    for ld in (vw, vw + 1):
+        dp, dlen = dev(pb), dev(np.zeros(B, np.int32))
+        dring, dstate = out_buf(B * ring * C * 2), out_buf(nslots * B * nv * dv * dk * 4)
+        dcw, dal, ddt, dnw = dev(c["cwb"]), dev(c["alb"]), dev(c["dtb"]), dev(c["nwb"])
+        dout = out_buf(B * T * ld * 2)
+        wsb = kern().hai_deltanet_prefill_workspace_bytes(B, T, nv, dv)
+        dws = out_buf(wsb)
+        hai.check(kern().hai_deltanet_prefill_bf16(dout.ptr, ld, dp.ptr, width, 0, C, C + vw, C + vw + nv, dcw.ptr,
+                                                   dring.ptr, ring, dstate.ptr, nslots, dal.ptr, ddt.ptr, dnw.ptr,
+                                                   dlen.ptr, 0, B, T, nk, nv, dk, dv, Kc, 1e-6, dws.ptr, wsb, None),
+                  "deltanet_prefill")
+        outs.append(dout.download(np.uint16).reshape(B * T, ld)[:, :vw].copy())
+    bad = outs[0] != outs[1]
+    assert not bad.any(), int(bad.sum())
+
+
 @pytest.mark.parametrize("B,nk,nv,dk,T,Kc,ab", [(3, 2, 6, 64, 40, 4, False), (2, 16, 48, 128, 33, 4, True),
                                                 (1, 4, 4, 64, 100, 3, False)])
 def test_deltanet_prompt_chunk_equals_16_token_launches(B, nk, nv, dk, T, Kc, ab):

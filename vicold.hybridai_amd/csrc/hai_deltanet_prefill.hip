@@ -675,8 +675,8 @@ __global__ __launch_bounds__(256) void deltanet_ring_update_kernel(uint16_t* __r
 }
 
 // Gated RMSNorm of the outputs: one wave per (row, head); rms of the
-// unrounded output, then bf16(((bf16(o) * rms) * w) * silu(z))
-// (the verify kernel's epilogue).
+// unrounded output, then bf16(((bf16(o) * rms) * w) * silu(z)) (the verify
+// kernel's epilogue, silu within 2^-21 of it).
 template <int DV>
 __global__ __launch_bounds__(256) void deltanet_gated_norm_kernel(uint16_t* __restrict__ out, int64_t ld_out,
                                                                   const float* __restrict__ o_ws,
@@ -696,16 +696,17 @@ __global__ __launch_bounds__(256) void deltanet_gated_norm_kernel(uint16_t* __re
     for (int r = 0; r < PER; ++r) {
         const int jo = lane + 64 * r;
         const float z = bf2f(proj[row * ld_proj + off_z + static_cast<int64_t>(h) * DV + jo]);
-        out[row * ld_out + static_cast<int64_t>(h) * DV + jo] = f2bf(((bfr(o[jo]) * rms) * bf2f(norm_w[jo])) * csilu(z));
+        out[row * ld_out + static_cast<int64_t>(h) * DV + jo] = f2bf(((bfr(o[jo]) * rms) * bf2f(norm_w[jo])) * hw_silu(z));
     }
 }
 
 // Both of the above in one launch with 16-byte accesses: the first nblocks
 // blocks take 256 / (DV / 8) head rows each (DV / 8 lanes a row), the rest the
 // ring's entries as dword pairs.  Needs 16-byte aligned rows of out, proj's z
-// columns and the norm weight.  Bound by memory (o in fp32, z, out); MI355X,
-// 1000 tokens of 48 heads: 20.4 + 4.6 -> 9.6 us (two bytes per lane, canonical
-// exp and IEEE division in the gate).
+// columns and the norm weight; the same sums and gate as the two-byte form, bit
+// for bit.  Bound by memory (o in fp32, z, out); MI355X, 1000 tokens of 48 heads:
+// 20.4 + 4.6 -> 9.6 us (two bytes per lane, canonical exp and IEEE division in
+// the gate, which here would take 4.5 us more).
 template <int DV>
 __global__ __launch_bounds__(256) void deltanet_gated_norm_ring_kernel(
     uint16_t* __restrict__ out, int64_t ld_out, const float* __restrict__ o_ws, const uint16_t* __restrict__ proj,
@@ -745,8 +746,8 @@ __global__ __launch_bounds__(256) void deltanet_gated_norm_ring_kernel(
     uint32_t y[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-        y[q] = f2bf2(((bfr(o[2 * q]) * rms) * lo_bf(nw[q])) * fast_silu(lo_bf(z[q])),
-                     ((bfr(o[2 * q + 1]) * rms) * hi_bf(nw[q])) * fast_silu(hi_bf(z[q])));
+        y[q] = f2bf2(((bfr(o[2 * q]) * rms) * lo_bf(nw[q])) * hw_silu(lo_bf(z[q])),
+                     ((bfr(o[2 * q + 1]) * rms) * hi_bf(nw[q])) * hw_silu(hi_bf(z[q])));
     *reinterpret_cast<u32x4*>(out + row * ld_out + static_cast<int64_t>(h) * DV + j0) = u32x4{y[0], y[1], y[2], y[3]};
 }
 

@@ -116,6 +116,7 @@ __device__ __forceinline__ float hw_sigmoid(float x) {
     const float e = __builtin_amdgcn_exp2f(x * -0x1.7154p+0f) * c;
     return __builtin_amdgcn_rcpf(fma_(e, 0x1p-64f, 0x1p-64f)) * 0x1p-64f;
 }
+__device__ __forceinline__ float hw_silu(float x) { return x * hw_sigmoid(x); }
 __device__ __forceinline__ float csqrt(float x) { return __builtin_sqrtf(x); }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
