@@ -1027,6 +1027,36 @@ def test_deltanet_prefill_norm_forms_agree():
     assert not bad.any(), int(bad.sum())
 
 
+def test_deltanet_prefill_output_over_projection_rows():
+    """Output rows written over the q columns of the projection rows: the conv
+    ring takes those columns' last rows before they are overwritten, so out,
+    ring and state equal those of a call with its own output, bit for bit."""
+    rng = np.random.default_rng(78)
+    B, T, nk, nv, dk, Kc, ring, nslots = 2, 70, 4, 4, 128, 4, 96, 80
+    dv = dk
+    vw, width = nv * dv, 2 * nk * dk + 2 * nv * dv + 16
+    c = _deltanet_case(rng, B, nk, nv, dk, dv, Kc)
+    C = c["C"]
+    _, pb = rand_bf16(rng, (B * T, width))
+    res = []
+    for own in (True, False):
+        dp, dlen = dev(pb), dev(np.zeros(B, np.int32))
+        dring, dstate = out_buf(B * ring * C * 2), out_buf(nslots * B * nv * dv * dk * 4)
+        dcw, dal, ddt, dnw = dev(c["cwb"]), dev(c["alb"]), dev(c["dtb"]), dev(c["nwb"])
+        dout = out_buf(B * T * vw * 2)
+        wsb = kern().hai_deltanet_prefill_workspace_bytes(B, T, nv, dv)
+        dws = out_buf(wsb)
+        hai.check(kern().hai_deltanet_prefill_bf16(dout.ptr if own else dp.ptr, vw if own else width, dp.ptr, width,
+                                                   0, C, C + vw, C + vw + nv, dcw.ptr, dring.ptr, ring, dstate.ptr,
+                                                   nslots, dal.ptr, ddt.ptr, dnw.ptr, dlen.ptr, 0, B, T, nk, nv, dk,
+                                                   dv, Kc, 1e-6, dws.ptr, wsb, None), "deltanet_prefill")
+        o = dout.download(np.uint16).reshape(B * T, vw) if own else \
+            dp.download(np.uint16).reshape(B * T, width)[:, :vw]
+        res.append((o.copy(), dring.download(np.uint16), dstate.download(np.uint32)))
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("B,nk,nv,dk,T,Kc,ab", [(3, 2, 6, 64, 40, 4, False), (2, 16, 48, 128, 33, 4, True),
                                                 (1, 4, 4, 64, 100, 3, False)])
 def test_deltanet_prompt_chunk_equals_16_token_launches(B, nk, nv, dk, T, Kc, ab):

@@ -765,6 +765,16 @@ int64_t device_cus() {
     return 256;  // MI355X
 }
 
+// Whether the address ranges of `rows` rows of width elements at out (pitch ld_out) and of as many at proj (pitch
+// ld_proj) meet.
+bool rows_overlap(const uint16_t* out, int64_t ld_out, int64_t width, const uint16_t* proj, int64_t ld_proj,
+                  int64_t rows) {
+    const uintptr_t o0 = reinterpret_cast<uintptr_t>(out), p0 = reinterpret_cast<uintptr_t>(proj);
+    const uintptr_t o1 = o0 + static_cast<uintptr_t>((rows - 1) * ld_out + width) * 2;
+    const uintptr_t p1 = p0 + static_cast<uintptr_t>(rows * ld_proj) * 2;
+    return o0 < p1 && p0 < o1;
+}
+
 template <int DK, int DV, int NWB>
 int launch_state(const PrefillArgs& a, hipStream_t s) {
     constexpr size_t shmem = StateShape<DK, DV, NWB>::LDS_BYTES;
@@ -803,7 +813,10 @@ int launch_prefill(const PrefillArgs& a, uint16_t* out, int64_t ld_out, int64_t 
     if (rc != HAI_OK) return rc;
     const int hist = a.Kc - 1;
     const int64_t tasks = static_cast<int64_t>(a.B) * a.T * a.nv;
-    if (aligned16(out) && ld_out % 8 == 0 && aligned16(a.proj) && a.ld_proj % 8 == 0 && off_z % 8 == 0 &&
+    // one launch for both, unless out lies among the projection rows: its blocks run in any order, and the ring's
+    // take the last rows' inputs, which the norm's would then overwrite
+    if (!rows_overlap(out, ld_out, static_cast<int64_t>(a.nv) * DV, a.proj, a.ld_proj, static_cast<int64_t>(a.B) * a.T) &&
+        aligned16(out) && ld_out % 8 == 0 && aligned16(a.proj) && a.ld_proj % 8 == 0 && off_z % 8 == 0 &&
         aligned16(norm_w)) {
         const int64_t C = 2 * static_cast<int64_t>(a.nk) * DK + static_cast<int64_t>(a.nv) * DV;
         const int64_t per = 256 / (DV / 8);
