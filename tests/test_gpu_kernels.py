@@ -1652,6 +1652,49 @@ def test_gemm_ring_rows_do_not_depend_on_the_row_count(fp8, N, K):
         assert np.array_equal(r, rows[0])
 
 
+@pytest.mark.parametrize("fp8,M", [(False, 32), (False, 64), (True, 64)])
+def test_gemm_ring_swiglu_every_bf16_gate(fp8, M):
+    """The ring-staged form's SwiGLU: one-hot rows pick the gate (and 1 as up)
+    out of the weights, so every output is silu(gate) rounded to bf16: half a
+    bf16 unit from float64 and 2^-21 of it for the fp32 arithmetic, down to where
+    the canonical silu's e^-gate overflows (bf16 weights: every bf16 gate; FP8:
+    every code times its scale)."""
+    K, F = 128, 1024
+    rng = np.random.default_rng(M)
+    x = np.zeros((M, K), np.float32)
+    x[np.arange(M), np.arange(M) % K] = 1.0
+    dx, dy = dev(hai.bf16_bits(x)), out_buf(M * F * 2)
+    if fp8:
+        codes = np.resize(np.arange(256, dtype=np.uint8), F * K).reshape(K, F).T.copy()
+        codes[(codes & 0x7F) == 0x7F] = 0
+        sg = (2.0 ** rng.integers(-3, -1, (F // 128, 1))).astype(np.float32)
+        q = np.empty((2 * F, K), np.uint8)
+        q[0::2], q[1::2] = codes, 0x38  # up = 1
+        s = np.stack([sg, np.ones_like(sg)])
+        g = orc.gemm_fp8(x, codes, sg)
+        dq, ds = dev(q), dev(s)
+        hai.check(kern().hai_gemm_fp8_mfma(dy.ptr, F, dx.ptr, K, dq.ptr, ds.ptr, None, M, 2 * F, K,
+                                           hai.EPI_SILU_MUL | hai.FP8_NO_SPECIAL_CODES, None, 0, None, 0, None), "fp8")
+    else:
+        gates = np.resize(np.arange(65536, dtype=np.uint16), M * F)
+        gates[~np.isfinite(hai.bf16_to_f32(gates))] = 0  # (times the other rows' zeros)
+        wb = np.zeros((2 * F, K), np.uint16)
+        wb[0::2, :M] = gates.reshape(M, F).T
+        wb[1::2, :M] = hai.bf16_bits(np.ones(1, np.float32))[0]
+        g = hai.bf16_to_f32(gates).reshape(M, F)
+        dw = dev(wb)
+        hai.check(kern().hai_gemm_bf16_mfma(dy.ptr, F, dx.ptr, K, dw.ptr, M, 2 * F, K, hai.EPI_SILU_MUL, None, 0,
+                                            None, 0, None), "bf16")
+    got = dy.download(np.uint16)
+    g = g.astype(np.float64)
+    with np.errstate(all="ignore"):
+        want = np.where(g < -88.72284, 0.0, g / (1.0 + np.exp(-g))).reshape(-1)
+    got = hai.bf16_to_f32(got).astype(np.float64)
+    unit = 2.0 ** (np.maximum(np.floor(np.log2(np.maximum(np.abs(want), 1e-300))), -126) - 7)
+    bad = np.abs(got - want) > 0.5 * unit + 2.0 ** -21 * np.abs(want)
+    assert not bad.any(), (int(bad.sum()), g.reshape(-1)[bad][:8], got[bad][:8], want[bad][:8])
+
+
 @pytest.mark.parametrize("M,N,K,epi", [(32, 34816, 5120, 2), (32, 5120, 17408, 1), (64, 16480, 5120, 0)])
 def test_gemm_mfma_27b_shapes(M, N, K, epi):
     """The batched-verify GEMMs at their C4 (M = 8 sequences x 4 rows) and C5

@@ -374,7 +374,7 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
                 const float g = bfr(tot[i]);
                 const float u = quad_xor1(g);
                 if ((lc & 1) == 0 && col && m < a.M)
-                    a.y[static_cast<int64_t>(m) * a.ldy + n / 2] = f2bf(fast_silu(g) * u);
+                    a.y[static_cast<int64_t>(m) * a.ldy + n / 2] = f2bf(hw_silu(g) * u);
             }
         } else if (col) {
 #pragma unroll

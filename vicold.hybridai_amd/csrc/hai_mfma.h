@@ -1,6 +1,5 @@
 // hai_mfma.h -- matrix-core primitives shared by the batched and prompt GEMMs:
-// the bf16 MFMA forms, the exact E4M3 -> bf16 decode, the tolerance-mode
-// SiLU.
+// the bf16 MFMA forms and the exact E4M3 -> bf16 decode.
 #pragma once
 
 #include "hai_device.h"
@@ -57,11 +56,6 @@ __device__ __forceinline__ uint32_t e4m3x2_to_bf16(uint32_t w, bool high) {
     const b2v v = high ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true)
                        : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, false);
     return __builtin_bit_cast(uint32_t, v);
-}
-
-// silu by the hardware exp2 and reciprocal (tolerance mode)
-__device__ __forceinline__ float fast_silu(float x) {
-    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
 }
 
 }  // namespace hai
