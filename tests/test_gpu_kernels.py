@@ -1652,6 +1652,38 @@ def test_gemm_ring_rows_do_not_depend_on_the_row_count(fp8, N, K):
         assert np.array_equal(r, rows[0])
 
 
+@pytest.mark.parametrize("fp8,N,K,splits", [
+    (True, 5120, 3840, 4), (True, 5120, 11008, 4), (False, 4096, 4352, 4),  # K / 256 not a multiple of the splits
+    (True, 8192, 4992, 4)])  # an odd number of 128-k chunks
+def test_gemm_split_rows_do_not_depend_on_the_row_count(fp8, N, K, splits):
+    """A row gives the same bits whether the call has 4 or 64 rows (a verify
+    and a correction of the same row round alike)."""
+    rng = np.random.default_rng(N + K)
+    x, xb = rand_bf16(rng, (64, K))
+    if fp8:
+        q, s = _fp8_weights(rng, N, K)
+        dw, ds = dev(q), dev(s)
+    else:
+        dw, ds = dev(rand_bf16(rng, (N, K), 0.05)[1]), None
+    dx = dev(xb)
+    rows = []
+    for M in (4, 16, 17, 32, 33, 64):
+        dy = out_buf(M * N * 2)
+        wsb = kern().hai_gemm_mfma_workspace_bytes(M, N)
+        dws = out_buf(max(wsb, 16))
+        if splits is not None:
+            assert kern().hai_gemm_mfma_splits(M, N, K, dws.ptr, wsb) == splits
+        if fp8:
+            hai.check(kern().hai_gemm_fp8_mfma(dy.ptr, N, dx.ptr, K, dw.ptr, ds.ptr, None, M, N, K,
+                                               hai.FP8_NO_SPECIAL_CODES, None, 0, dws.ptr, wsb, None), "fp8 mfma")
+        else:
+            hai.check(kern().hai_gemm_bf16_mfma(dy.ptr, N, dx.ptr, K, dw.ptr, M, N, K, 0, None, 0, dws.ptr, wsb,
+                                                None), "bf16 mfma")
+        rows.append(dy.download(np.uint16).reshape(M, N)[:4])
+    for i, r in enumerate(rows[1:]):
+        assert np.array_equal(r, rows[0]), (i, int((r != rows[0]).sum()))
+
+
 @pytest.mark.parametrize("fp8,M", [(False, 32), (False, 64), (True, 64)])
 def test_gemm_ring_swiglu_every_bf16_gate(fp8, M):
     """The ring-staged form's SwiGLU: one-hot rows pick the gate (and 1 as up)

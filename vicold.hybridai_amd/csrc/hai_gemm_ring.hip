@@ -1,5 +1,6 @@
 // hai_gemm_ring.hip -- batched-verify linear layer, ring-staged form (see
 // hai_gemm_mfma.hip for the contract and the other forms).
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -118,7 +119,6 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
     const int lane = threadIdx.x & 63;
     const int wave = wave_index();
     const int lc = lane & 31, lh = lane >> 5;
-    const int nck = a.K / (KC * kRingK);  // steps of KC chunks
     const int R = a.R;
     const int wstage = SH::w_stage(R);
     const uint32_t lds0 = static_cast<uint32_t>(
@@ -128,11 +128,17 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
     // FP8, 178 MB, M = 32: 47.7 -> 42.1 us with the norm; 16384 x 5120, 84 MB: 24.2 -> 24.8)
     const bool nt = static_cast<int64_t>(a.N) * a.K * SH::EB > (int64_t{96} << 20);
     const int items = a.tiles * a.splits;
-    auto chunk_lo = [&](int split) { return static_cast<int>(static_cast<int64_t>(split) * nck / a.splits); };
-    // total chunks of this block
+    // first step (of KC chunks) of a split: K is cut between pairs of chunks whatever KC is, so that a row's sums do
+    // not depend on the form that the number of rows selects
+    const int nck = a.K / kRingK;
+    auto step_lo = [&](int split) {
+        const int pair = static_cast<int>(static_cast<int64_t>(split) * ((nck + 1) / 2) / a.splits);
+        return KC == 2 ? pair : min(2 * pair, nck);
+    };
+    // total steps of this block
     int total = 0;
     for (int it = blockIdx.x; it < items; it += gridDim.x)
-        total += chunk_lo(it / a.tiles + 1) - chunk_lo(it / a.tiles);
+        total += step_lo(it / a.tiles + 1) - step_lo(it / a.tiles);
 
     if (wave >= NG * MT) {  // ---- a copying wave: weights and scales ----
         const int p = wave - NG * MT;
@@ -147,8 +153,8 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
         auto open_item = [&]() {  // (item < items)
             const int tile = item % a.tiles;
             const int split = item / a.tiles;
-            c = chunk_lo(split);
-            cend = chunk_lo(split + 1);
+            c = step_lo(split);
+            cend = step_lo(split + 1);
             const int64_t row0 = static_cast<int64_t>(tile) * R;
             last = static_cast<int>(min(static_cast<int64_t>(R), a.N - row0)) - 1;
             wbase = static_cast<const char*>(a.w) + row0 * a.K * SH::EB;
@@ -249,7 +255,7 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
                   (((lane % XLANES) ^ SH::x_swz(r)) << 4);
         xdst[j] = __builtin_amdgcn_readfirstlane(ldsx + i * 1024);
     }
-    int xitem = blockIdx.x, xc = chunk_lo(xitem / a.tiles), xend = chunk_lo(xitem / a.tiles + 1), xslot = 0, xasked = 0;
+    int xitem = blockIdx.x, xc = step_lo(xitem / a.tiles), xend = step_lo(xitem / a.tiles + 1), xslot = 0, xasked = 0;
     auto request_x = [&]() {
         const void* xb = uniform_ptr(reinterpret_cast<const char*>(a.x) + static_cast<int64_t>(xc) * SH::XROW);
 #pragma unroll
@@ -260,8 +266,8 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
         if (++xc == xend) {
             xitem += gridDim.x;
             if (xitem < items) {
-                xc = chunk_lo(xitem / a.tiles);
-                xend = chunk_lo(xitem / a.tiles + 1);
+                xc = step_lo(xitem / a.tiles);
+                xend = step_lo(xitem / a.tiles + 1);
             }
         }
     };
@@ -270,11 +276,11 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
     for (int item = blockIdx.x; item < items; item += gridDim.x) {
         const int tile = item % a.tiles;
         const int split = item / a.tiles;
-        const int cend = chunk_lo(split + 1);
+        const int cend = step_lo(split + 1);
         f32x16 tot;
 #pragma unroll
         for (int i = 0; i < 16; ++i) tot[i] = 0.0f;
-        for (int c = chunk_lo(split); c < cend; ++c) {
+        for (int c = step_lo(split); c < cend; ++c) {
             // this wave's copies of the chunk have landed, then everyone's
             if (done + SX - 2 < total) wait_vmcnt<(SX - 2) * SH::XCOPIES>();
             else wait_vmcnt<0>();
@@ -453,7 +459,8 @@ void ring_plan(RingArgs& r, int max_splits, bool fixed, int cus) {
             if (ring_stages(R, mt, fp8, ring_kc(R, M, r.K, fp8)) < 3) break;
             const int64_t tiles = (static_cast<int64_t>(r.N) + R - 1) / R;
             const int64_t rounds = (tiles * splits + cus - 1) / cus;
-            const double c = static_cast<double>(rounds) * static_cast<double>((nck + splits - 1) / splits) *
+            const int64_t chunks = std::min((((nck + 1) / 2 + splits - 1) / splits) * 2, nck);  // of the longest split
+            const double c = static_cast<double>(rounds) * static_cast<double>(chunks) *
                              (R * kRingK * eb + mt * 32 * kRingK * 2);
             if (best == 0 || c < cost) {
                 best = R;
