@@ -1,6 +1,5 @@
 // hai_gemm_ring.hip -- batched-verify linear layer, ring-staged form (see
 // hai_gemm_mfma.hip for the contract and the other forms).
-#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -459,8 +458,7 @@ void ring_plan(RingArgs& r, int max_splits, bool fixed, int cus) {
             if (ring_stages(R, mt, fp8, ring_kc(R, M, r.K, fp8)) < 3) break;
             const int64_t tiles = (static_cast<int64_t>(r.N) + R - 1) / R;
             const int64_t rounds = (tiles * splits + cus - 1) / cus;
-            const int64_t chunks = std::min((((nck + 1) / 2 + splits - 1) / splits) * 2, nck);  // of the longest split
-            const double c = static_cast<double>(rounds) * static_cast<double>(chunks) *
+            const double c = static_cast<double>(rounds) * static_cast<double>((nck + splits - 1) / splits) *
                              (R * kRingK * eb + mt * 32 * kRingK * 2);
             if (best == 0 || c < cost) {
                 best = R;
