@@ -555,7 +555,8 @@ int hai_correction_commit_bf16(const int32_t* result, const int64_t* corr_next,
  * K % 8 == 0, M <= 128.
  * workspace (may be NULL) lets narrow layers split K across blocks; with
  * hai_gemm_mfma_workspace_bytes(M, N) bytes every split is available, with
- * less the call uses fewer splits.  The result does not depend on it. */
+ * less the call uses fewer splits: the result then differs by the grouping
+ * of its fp32 sums only. */
 size_t hai_gemm_mfma_workspace_bytes(int64_t M, int64_t N);
 /* The FP8 block-scaled Linear (arguments as hai_gemm_fp8_bf16, K % 16 == 0)
  * on the matrix cores for M up to 128: codes decoded exactly to bf16, each
@@ -593,7 +594,10 @@ int hai_gemm_fp8_tiled(void* y, int64_t ldy, const void* x, int64_t ldx,
  * caller completes y = res (in place) with hai_mfma_residual_rmsnorm_bf16.
  * With one split the call finishes y itself. */
 enum { HAI_MFMA_KEEP_PARTIALS = 0x200 };
-/* The number of K splits the MFMA GEMM takes for this shape and workspace. */
+/* The number of K splits that a GEMM called with HAI_MFMA_KEEP_PARTIALS takes
+ * for this shape and workspace, and for N <= 8192 (where the partials can be
+ * completed by the call below) also the plain residual GEMM; the other
+ * epilogues and wider layers take at most as many. */
 int hai_gemm_mfma_splits(int64_t M, int64_t N, int64_t K, const void* workspace,
                          size_t workspace_bytes);
 /* Completes a residual MFMA GEMM called with HAI_MFMA_KEEP_PARTIALS, fused

@@ -1841,6 +1841,14 @@ def test_mfma_keep_partials_then_residual_rmsnorm(M, N, K, fp8):
                                              None, 0, dws.ptr, wsb, None) == hai.ERR_INVALID
 
 
+@pytest.mark.parametrize("M,N,K,fp8", [(20, 2560, 2688, False), (40, 6656, 3840, False), (64, 7616, 4224, False),
+                                       (8, 2560, 2688, True)])
+def test_mfma_kept_and_plain_residual_take_the_same_splits(M, N, K, fp8):
+    """Shapes where the ring-staged kernel's plan depends on the weight format:
+    the residual call follows hai_gemm_mfma_splits, kept or not."""
+    test_mfma_keep_partials_then_residual_rmsnorm(M, N, K, fp8)
+
+
 @pytest.mark.parametrize("M,N,K,fp8", [(32, 5120, 6144, False), (32, 5120, 17408, False), (64, 5120, 17408, True),
                                        (17, 1536, 4096, False), (128, 5120, 2048, True)])
 def test_mfma_fp32_accumulators_within_1e3(M, N, K, fp8):

@@ -999,7 +999,9 @@ int launch_ring_mfma(const MfmaArgs& a, hipStream_t s) {
     r.K = a.K;
     r.part = a.part;
     r.epi = EPI;
-    ring_plan(r, a.KSB, a.keep, device_cus());
+    // a kept call takes exactly the splits that hai_gemm_mfma_splits names, and so does the residual call that it
+    // equals bit for bit; the others, whose caller names no count, plan by the weight format
+    ring_plan(r, a.KSB, a.keep || (EPI == HAI_EPI_RESIDUAL && a.N <= kMaxResidualNormCols), device_cus());
     const int rc = launch_ring(r, a.check, device_cus(), s);
     if (rc != HAI_OK || r.splits == 1 || a.keep) return rc;
     const int64_t n = static_cast<int64_t>(a.M) * ((a.N + 1) / 2);
@@ -1071,7 +1073,7 @@ int choose_splits(int64_t M, int64_t N, int64_t K, const void* workspace, size_t
                workspace_bytes >= static_cast<size_t>(ksb * M * N) * sizeof(float);
     };
     if (N <= 8192 && ring_shape(M, K)) {
-        // the ring-staged kernel's own plan (the same for bf16 and FP8 weights)
+        // the ring-staged kernel's plan, at FP8 prices: the caller of hai_gemm_mfma_splits names no format
         static const float fp8_plan = 1.0f;
         int most = 4;
         while (most > 1 && !fits(most)) --most;

@@ -443,9 +443,9 @@ namespace hai {
 // 242 tiles of 144 rows, W alone 34 us, X alone 17, both 48).  A split adds its
 // partial planes and a second pass (about 9 us with its launch: 16384 x 5120 at
 // M = 64, 256 tiles of 64 33.5 us, 128 tiles of 128 in two splits 36.2).
-// The splits follow N, K and the weight format alone (priced for 64 rows), so
-// that a row's sums are the same whatever the number of rows: a verify and a
-// correction of the same row round alike.
+// The splits follow N, K, the weight format and the epilogue alone (priced for
+// 64 rows), so that a row's sums are the same whatever the number of rows: a
+// verify and a correction of the same row round alike.
 void ring_plan(RingArgs& r, int max_splits, bool fixed, int cus) {
     const bool fp8 = r.scales != nullptr;
     const int eb = fp8 ? 1 : 2;
