@@ -1010,17 +1010,17 @@ int launch_ring_mfma(const MfmaArgs& a, hipStream_t s) {
     return launched("mfma_finalize_kernel");
 }
 
-// The copy-staged kernel keeps the FP8 layers whose 64-row tiles load 3/4 to
-// 15/16 of the CUs (q|gate|k|v of the 27B shape, 224 tiles), where the ring
-// plan halves K for balance and pays the second pass: MI355X, 14336 x 5120 with
-// the RMSNorm before it, copy-staged / ring: M = 20 23.8 / 25.9 us, M = 32 23.0 /
-// 25.8, M = 48 30.9 / 30.3, M = 64 32.2 / 31.6.  Beside that range the ring is as
-// fast or faster (16384: M = 64 34.6 / 30.5, M = 32 23.6 / 24.1; 12288: 31.5 / 26.7
-// and 22.4 / 21.7).
+// The copy-staged kernel keeps the FP8 layers of short K whose 64-row tiles load
+// 3/4 to 15/16 of the CUs: it starts faster, the ring streams faster.  MI355X,
+// copy-staged / ring at 8, 32 and 64 rows: 14336 x 2048 10.1 / 11.1, 11.0 / 11.9,
+// 15.7 / 14.3 us, 12800 x 3072 13.7 / 14.5, 15.0 / 15.8, 20.8 / 18.5, 14336 x 4096
+// 17.4 / 18.0, 18.9 / 19.2, 25.6 / 23.8, 14336 x 5120 21.2 / 20.2, 23.0 / 23.2, 32.0 /
+// 27.9, 14336 x 8192 30.2 / 27.7, 32.4 / 29.7, 46.4 / 40.4.  The line does not follow
+// M, so that a row rounds alike in calls of any size.
 bool use_dma(const MfmaArgs& a) {
     const int64_t cus = device_cus();
     const int64_t ntiles = (static_cast<int64_t>(a.N) + kBlockRows - 1) / kBlockRows;
-    return a.wq != nullptr && a.K % kRtChunk == 0 && a.M > 16 && a.M <= 64 && a.N > 8192 && !a.keep &&
+    return a.wq != nullptr && a.K % kRtChunk == 0 && a.K < 4096 && a.M <= kRingMaxRows && a.N > 8192 && !a.keep &&
            4 * ntiles > 3 * cus && 16 * ntiles <= 15 * cus;
 }
 

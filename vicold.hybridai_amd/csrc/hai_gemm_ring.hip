@@ -443,6 +443,11 @@ namespace hai {
 // 242 tiles of 144 rows, W alone 34 us, X alone 17, both 48).  A split adds its
 // partial planes and a second pass (about 9 us with its launch: 16384 x 5120 at
 // M = 64, 256 tiles of 64 33.5 us, 128 tiles of 128 in two splits 36.2).
+// Wide FP8 layers are not split into tiles too tall for two chunks per step
+// (more than 96 rows): MI355X, one / two splits at 8, 32 and 64 rows, 14336 x
+// 5120 19.9 / 21.6, 23.0 / 23.2, 28.5 / 29.9 us, 16480 x 5120 21.1 / 23.6, 24.4 /
+// 26.3, 32.5 / 33.6; where the tiles stay shorter two win, 12288 x 5120 20.3 / 17.7,
+// 22.5 / 19.7, 26.4 / 26.9.
 // The splits follow N, K, the weight format and the epilogue alone (priced for
 // 64 rows), so that a row's sums are the same whatever the number of rows: a
 // verify and a correction of the same row round alike.
@@ -471,7 +476,8 @@ void ring_plan(RingArgs& r, int max_splits, bool fixed, int cus) {
     double cost = 0.0;
     for (int splits = 1; splits <= max_splits && !fixed; ++splits) {
         double c = 0.0;
-        best_tile(kRingMaxRows, splits, c);
+        const int R = best_tile(kRingMaxRows, splits, c);
+        if (splits > 1 && fp8 && r.N > 8192 && ring_kc(R, 1, r.K, fp8) == 1) continue;
         if (splits > 1) c += 270e3 + 8.0 * splits * kRingMaxRows * r.N / cus;
         if (splits == 1 || c < cost) {
             r.splits = splits;
