@@ -1624,6 +1624,19 @@ def test_gemm_ring_edges(fp8, M, N, K, epi, mapped):
         test_gemm_mfma_within_tolerance(M, N, K, epi, True)
 
 
+@pytest.mark.parametrize("fp8,M,N,K,epi,mapped", [
+    (True, 1, 4133, 2944, 0, True),  # three 32-row tiles per block, the last rows ragged
+    (True, 32, 96, 4224, 1, False),  # K split, the half step in the last split
+    (True, 20, 2 * 9000, 640, 2, False),  # several items per block: a half step between two tiles
+    (True, 16, 12345, 896, 0, False),  # 96-row tiles
+    (False, 1, 4133, 2944, 0, False), (False, 32, 96, 4224, 1, False), (False, 20, 2 * 9000, 640, 2, False)])
+def test_gemm_ring_odd_chunks(fp8, M, N, K, epi, mapped):
+    """Odd numbers of 128-k chunks up to 32 rows: steps of two chunks whose last
+    one holds a single chunk, same bounds as test_gemm_ring_edges (weights and
+    scales end with the tensor, so a read past the chunk would leave it)."""
+    test_gemm_ring_edges(fp8, M, N, K, epi, mapped)
+
+
 @pytest.mark.parametrize("fp8,N,K", [(True, 5120, 2048), (True, 9000, 768), (False, 5120, 2048), (False, 9000, 640)])
 def test_gemm_ring_rows_do_not_depend_on_the_row_count(fp8, N, K):
     """A row gives the same bits whether the call has 4, 32, 33 or 64 rows

@@ -867,11 +867,7 @@ int device_cus();
 // 64 80.5 / 55.6, M = 32 55 / 45, M = 4 44.6 / 44.6; bf16 M = 32 75 / 61, M = 64
 // 95 / 67; 16384 x 5120 FP8 35 / 32, bf16 M = 64 47 / 40; 5120 x 8192 FP8 27.8 /
 // 25.1; 8192 x 1024 17.5 / 12.5.  (Closest: 16384 x 5120 FP8 at 17-32 rows, 23.6
-// / 24.1.)  An odd number of chunks leaves one per step, which one computing
-// wave per block does not hide up to 32 rows, while from 33 rows on the ring
-// is ahead: LDS-staged / ring, 5568 x 2944 FP8 M = 5 16.6 / 18.6, M = 28 16.1 /
-// 18.4, M = 64 20.6 / 19.0 (bf16 21.7 / 19.0), 8192 x 4992 FP8 M = 32 20.8 /
-// 18.6.  The line does not follow M, so that a row rounds alike in calls of
+// / 24.1.)  The line does not follow M, so that a row rounds alike in calls of
 // any size.  K not a multiple of 128 and 65-128 rows keep the kernels here.
 bool ring_shape(int64_t M, int64_t K) { return K % kRingK == 0 && M <= kRingMaxRows; }
 

@@ -58,8 +58,12 @@ int ring_stages(int R, int mt, bool fp8, int kc) {
 }
 
 // Chunks per step.  Two where one chunk is too little work between barriers:
-// up to 32 rows (one computing wave per 32 weight rows) and short tiles.
-int ring_kc(int R, int M, int K, bool fp8) { return M <= 32 && R <= (fp8 ? 96 : 64) && K % (2 * kRingK) == 0 ? 2 : 1; }
+// up to 32 rows (one computing wave per 32 weight rows) and short tiles.  The
+// last step of an odd number of chunks holds its one chunk twice and takes the
+// first copy (MI355X, one chunk per step / this, 8 rows FP8: 1024 x 1152 8.2 / 7.3
+// us, 5568 x 4992 14.2 / 12.8, 5568 x 8320 18.1 / 15.9; 32 rows: 5568 x 4992 14.7 /
+// 13.6, 14336 x 5248 22.7 / 23.8).
+int ring_kc(int R, int M, int K, bool fp8) { return M <= 32 && R <= (fp8 ? 96 : 64) && K >= 2 * kRingK ? 2 : 1; }
 
 template <int MT, int NG, bool FP8, int KC>
 struct RingShape {
@@ -134,6 +138,7 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
         const int pair = static_cast<int>(static_cast<int64_t>(split) * ((nck + 1) / 2) / a.splits);
         return KC == 2 ? pair : min(2 * pair, nck);
     };
+    auto half_step = [&](int step) { return KC == 2 && 2 * step + 1 == nck; };  // a step of one chunk, held twice
     // total steps of this block
     int total = 0;
     for (int it = blockIdx.x; it < items; it += gridDim.x)
@@ -175,12 +180,17 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
         constexpr int PH = 4;
         const int ncopy = R / (WL * kRingCopiers);
         const uint32_t wpitch = static_cast<uint32_t>(a.K) * SH::EB;
+        constexpr int HALF_ROW = SH::WROW / 2;  // the second chunk's bytes of a row (KC = 2)
         uint32_t woff[PH];
 #pragma unroll
         for (int u = 0; u < PH; ++u)
             woff[u] = wr * wpitch + ((wpos ^ SH::w_swz((p + kRingCopiers * u) * WL + wr)) << 4);
-        auto copy_w = [&](auto stream, const void* wb, uint32_t dst) {
+        auto copy_w = [&](auto stream, const void* wb, uint32_t dst, bool half) {
             constexpr bool NT = decltype(stream)::value;
+            uint32_t wo[PH];  // (half: the second chunk's pieces repeat the first's)
+#pragma unroll
+            for (int u = 0; u < PH; ++u)
+                wo[u] = woff[u] - (half ? ((wpos ^ SH::w_swz((p + kRingCopiers * u) * WL + wr)) << 4) & HALF_ROW : 0);
             if (last == R - 1) {
                 const char* base = static_cast<const char*>(wb) + static_cast<int64_t>(p * WL) * wpitch;
                 const int64_t step = static_cast<int64_t>(kRingCopiers * WL) * wpitch;
@@ -189,8 +199,8 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
 #pragma unroll
                     for (int u = 0; u < PH; ++u) {
                         if (t + u >= ncopy) break;
-                        if constexpr (NT) ring_copy16_nt(woff[u], base, dst);
-                        else ring_copy16(woff[u], base, dst);
+                        if constexpr (NT) ring_copy16_nt(wo[u], base, dst);
+                        else ring_copy16(wo[u], base, dst);
                         base += step;
                         dst += kRingCopiers * 1024;
                     }
@@ -199,7 +209,9 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
                 for (int t = 0; t < ncopy; ++t) {
                     const int i = p + kRingCopiers * t;
                     const int r = i * WL + wr;
-                    const uint32_t off = static_cast<uint32_t>(min(r, last)) * wpitch + ((wpos ^ SH::w_swz(r)) << 4);
+                    const uint32_t piece = static_cast<uint32_t>(wpos ^ SH::w_swz(r)) << 4;
+                    const uint32_t off =
+                        static_cast<uint32_t>(min(r, last)) * wpitch + (half ? piece & ~static_cast<uint32_t>(HALF_ROW) : piece);
                     if constexpr (NT) ring_copy16_nt(off, wb, dst + i * 1024);
                     else ring_copy16(off, wb, dst + i * 1024);
                 }
@@ -208,13 +220,16 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
         auto request = [&]() {  // the cursor's chunk into the next slot
             const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + slot * wstage);
             const void* wb = uniform_ptr(wbase + static_cast<int64_t>(c) * SH::WROW);
-            if (nt) copy_w(std::true_type{}, wb, dst);
-            else copy_w(std::false_type{}, wb, dst);
+            const bool half = half_step(c);
+            if (nt) copy_w(std::true_type{}, wb, dst, half);
+            else copy_w(std::false_type{}, wb, dst, half);
             if constexpr (FP8) {
 #pragma unroll
-                for (int i = 0; i < SH::SCALE_COPIES; ++i)
-                    ring_copy4(srow[i] + c * (4 * KC), a.scales,
-                               dst + R * SH::WROW + min(p + kRingCopiers * i, KC * NG - 1) * 256);
+                for (int i = 0; i < SH::SCALE_COPIES; ++i) {
+                    const int g = min(p + kRingCopiers * i, KC * NG - 1);
+                    ring_copy4(srow[i] + c * (4 * KC) - (half ? 4 * (g % KC) : 0), a.scales,
+                               dst + R * SH::WROW + g * 256);
+                }
             }
             slot = slot + 1 == SW ? 0 : slot + 1;
             if (++c == cend) {
@@ -257,9 +272,16 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
     int xitem = blockIdx.x, xc = step_lo(xitem / a.tiles), xend = step_lo(xitem / a.tiles + 1), xslot = 0, xasked = 0;
     auto request_x = [&]() {
         const void* xb = uniform_ptr(reinterpret_cast<const char*>(a.x) + static_cast<int64_t>(xc) * SH::XROW);
+        if (half_step(xc)) {  // the second chunk's pieces (the permutation leaves their bit alone) repeat the first's
 #pragma unroll
-        for (int j = 0; j < SH::XCOPIES; ++j)
-            ring_copy16(xoff[j], xb, __builtin_amdgcn_readfirstlane(xdst[j] + xslot * SH::XB));
+            for (int j = 0; j < SH::XCOPIES; ++j)
+                ring_copy16(xoff[j] - (((lane % XLANES) & (XLANES / 2)) << 4), xb,
+                            __builtin_amdgcn_readfirstlane(xdst[j] + xslot * SH::XB));
+        } else {
+#pragma unroll
+            for (int j = 0; j < SH::XCOPIES; ++j)
+                ring_copy16(xoff[j], xb, __builtin_amdgcn_readfirstlane(xdst[j] + xslot * SH::XB));
+        }
         xslot = xslot + 1 == SX ? 0 : xslot + 1;
         ++xasked;
         if (++xc == xend) {
@@ -343,13 +365,16 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int q = 0; q < KC; ++q)
+                for (int q = 0; q < KC; ++q) {
+                    if (q > 0 && half_step(c)) break;
 #pragma unroll
                     for (int i = 0; i < 16; ++i) tot[i] = fma_(sc[q], acc[q][i], tot[i]);
+                }
             } else {
                 u32x4 wb[8], xa[8];
 #pragma unroll
                 for (int q = 0; q < KC; ++q) {
+                    if (q > 0 && half_step(c)) break;
 #pragma unroll
                     for (int t = 0; t < 8; ++t) {
                         wb[t] = ring_read16(w0 + so + (((16 * q + 2 * t + lh) ^ wsw) << 4));
