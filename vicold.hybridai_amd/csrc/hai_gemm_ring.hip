@@ -114,7 +114,7 @@ __device__ __forceinline__ void ring_copy4(uint32_t off, const void* base, uint3
 __device__ __forceinline__ u32x4 ring_read16(uint32_t lds) {
     return *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)lds;
 }
-template <int MT, int NG, bool FP8, bool CHECK, int KC>
+template <int MT, int NG, bool FP8, bool CHECK, int KC, bool ODD>
 __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_kernel(RingArgs a, int SW) {
     using SH = RingShape<MT, NG, FP8, KC>;
     constexpr int SX = SH::SX;
@@ -138,7 +138,9 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
         const int pair = static_cast<int>(static_cast<int64_t>(split) * ((nck + 1) / 2) / a.splits);
         return KC == 2 ? pair : min(2 * pair, nck);
     };
-    auto half_step = [&](int step) { return KC == 2 && 2 * step + 1 == nck; };  // a step of one chunk, held twice
+    // a step of one chunk, held twice (ODD: an odd number of chunks; an instance of its own, the tests cost the even
+    // ones up to 10 %)
+    auto half_step = [&](int step) { return KC == 2 && ODD && 2 * step + 1 == nck; };
     // total steps of this block
     int total = 0;
     for (int it = blockIdx.x; it < items; it += gridDim.x)
@@ -419,13 +421,13 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
     }
 }
 
-template <int MT, int NG, bool FP8, bool CHECK, int KC = 1>
+template <int MT, int NG, bool FP8, bool CHECK, int KC = 1, bool ODD = false>
 int launch_ring_as(const RingArgs& r, int cus, hipStream_t s) {
     using SH = RingShape<MT, NG, FP8, KC>;
     static std::atomic<uint8_t> allowed[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return invalid("gemm_mfma: device");
-    auto* kern = gemm_ring_mfma_kernel<MT, NG, FP8, CHECK, KC>;
+    auto* kern = gemm_ring_mfma_kernel<MT, NG, FP8, CHECK, KC, ODD>;
     if (!allowed[dev].load(std::memory_order_acquire)) {
         const int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds),
@@ -440,14 +442,19 @@ int launch_ring_as(const RingArgs& r, int cus, hipStream_t s) {
     kern<<<dim3(grid), dim3(64 * SH::WAVES), shmem, s>>>(r, sw);
     return launched("gemm_ring_mfma_kernel");
 }
+template <int MT, bool FP8, bool CHECK, bool ODD>  // two chunks per step
+int launch_ring_pairs(const RingArgs& r, int cus, hipStream_t s) {
+    if (r.R <= 32) return launch_ring_as<MT, 1, FP8, CHECK, 2, ODD>(r, cus, s);
+    if constexpr (FP8)
+        if (r.R > 64) return launch_ring_as<MT, 3, FP8, CHECK, 2, ODD>(r, cus, s);
+    return launch_ring_as<MT, 2, FP8, CHECK, 2, ODD>(r, cus, s);
+}
 template <int MT, bool FP8, bool CHECK>
 int launch_ring_ng(const RingArgs& r, int cus, hipStream_t s) {
     if constexpr (MT == 1) {
-        if (ring_kc(r.R, r.M, r.K, FP8) == 2) {
-            if (r.R <= 32) return launch_ring_as<MT, 1, FP8, CHECK, 2>(r, cus, s);
-            if (r.R <= 64) return launch_ring_as<MT, 2, FP8, CHECK, 2>(r, cus, s);
-            if constexpr (FP8) return launch_ring_as<MT, 3, FP8, CHECK, 2>(r, cus, s);
-        }
+        if (ring_kc(r.R, r.M, r.K, FP8) == 2)
+            return r.K / kRingK % 2 != 0 ? launch_ring_pairs<MT, FP8, CHECK, true>(r, cus, s)
+                                         : launch_ring_pairs<MT, FP8, CHECK, false>(r, cus, s);
     }
     switch ((r.R + 31) / 32) {
         case 1: return launch_ring_as<MT, 1, FP8, CHECK>(r, cus, s);
