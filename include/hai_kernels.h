@@ -594,10 +594,9 @@ int hai_gemm_fp8_tiled(void* y, int64_t ldy, const void* x, int64_t ldx,
  * caller completes y = res (in place) with hai_mfma_residual_rmsnorm_bf16.
  * With one split the call finishes y itself. */
 enum { HAI_MFMA_KEEP_PARTIALS = 0x200 };
-/* The number of K splits that a GEMM called with HAI_MFMA_KEEP_PARTIALS takes
- * for this shape and workspace, and for N <= 8192 (where the partials can be
- * completed by the call below) also the plain residual GEMM; the other
- * epilogues and wider layers take at most as many. */
+/* The number of K splits the MFMA GEMM takes for this shape and workspace
+ * (above N = 8192, where no call completes kept partials, a plain call takes at
+ * most as many). */
 int hai_gemm_mfma_splits(int64_t M, int64_t N, int64_t K, const void* workspace,
                          size_t workspace_bytes);
 /* Completes a residual MFMA GEMM called with HAI_MFMA_KEEP_PARTIALS, fused

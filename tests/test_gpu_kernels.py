@@ -1667,8 +1667,10 @@ def test_gemm_ring_rows_do_not_depend_on_the_row_count(fp8, N, K):
 
 @pytest.mark.parametrize("fp8,N,K,splits", [
     (True, 5120, 3840, 4), (True, 5120, 11008, 4), (False, 4096, 4352, 4),  # K / 256 not a multiple of the splits
-    (True, 8192, 4992, 4),  # an odd number of 128-k chunks
-    (True, 14336, 5120, None), (True, 14336, 1024, None)])  # wide layers: ring-staged without a split, copy-staged
+    (True, 8192, 4992, 2),  # an odd number of 128-k chunks
+    (True, 14336, 5120, None), (True, 14336, 1024, None),  # wide layers: ring-staged without a split, copy-staged
+    (False, 1536, 2560, 4), (True, 1536, 2560, 4), (True, 5120, 2048, 3), (True, 9000, 768, 1),  # small layers
+    (False, 8192, 2176, 2)])
 def test_gemm_split_rows_do_not_depend_on_the_row_count(fp8, N, K, splits):
     """A row gives the same bits whether the call has 4 or 64 rows (a verify
     and a correction of the same row round alike)."""

@@ -862,14 +862,30 @@ struct MfmaArgs {
 
 int device_cus();
 
-// The shapes that the ring-staged kernel takes: every one it can.  MI355X, us
-// with the RMSNorm before it, the kernels it replaced / ring: gate|up FP8 M =
-// 64 80.5 / 55.6, M = 32 55 / 45, M = 4 44.6 / 44.6; bf16 M = 32 75 / 61, M = 64
-// 95 / 67; 16384 x 5120 FP8 35 / 32, bf16 M = 64 47 / 40; 5120 x 8192 FP8 27.8 /
-// 25.1; 8192 x 1024 17.5 / 12.5.  (Closest: 16384 x 5120 FP8 at 17-32 rows, 23.6
-// / 24.1.)  The line does not follow M, so that a row rounds alike in calls of
-// any size.  K not a multiple of 128 and 65-128 rows keep the kernels here.
+// The shapes that the ring-staged kernel can take; it takes them but for those
+// of lds_shape and use_dma.  MI355X, us with the RMSNorm before it, the kernels it
+// replaced / ring: gate|up FP8 M = 64 80.5 / 55.6, M = 32 55 / 45, M = 4 44.6 / 44.6;
+// bf16 M = 32 75 / 61, M = 64 95 / 67; 16384 x 5120 FP8 35 / 32, bf16 M = 64 47 / 40;
+// 5120 x 8192 FP8 27.8 / 25.1.  (Closest: 16384 x 5120 FP8 at 17-32 rows, 23.6 /
+// 24.1.)  None of the lines follows M, so that a row rounds alike in calls of up
+// to 64 rows.  K not a multiple of 128 and 65-128 rows keep the kernels here.
 bool ring_shape(int64_t M, int64_t K) { return K % kRingK == 0 && M <= kRingMaxRows; }
+
+// Layers whose weights pass in a few us, much of it the start of the launch: the
+// splits are those that load the CUs evenly.
+bool small_layer(int64_t N, int64_t K) { return N <= 8192 && K <= 8192 && N * K <= (int64_t{1} << 24); }
+
+// Of the ring's shapes, those that the LDS-staged kernel keeps, because its
+// blocks start faster: walks too short to be split, in at most one 64-row tile
+// per CU (MI355X, ring / LDS-staged at 4, 32 and 64 rows: 8192 x 512 FP8 6.1 / 4.9,
+// 9.9 / 5.9, 10.6 / 8.1 us, 16384 x 768 FP8 7.5 / 6.5, 8.8 / 7.9, 9.6 / 10.3, 12288 x 512
+// bf16 7.5 / 5.2, 10.7 / 6.0, 12.1 / 8.3; 34816 x 512 9.7 / 11.9, 12.9 / 16.2, 17.7 /
+// 16.9), and small bf16 layers (4, 32 and 64 rows: 1024 x 2944 10.6 / 8.5, 9.9 / 8.9,
+// 10.8 / 11.6, 4096 x 2048 11.4 / 9.0, 13.1 / 10.2, 15.2 / 12.2, 2048 x 6144 13.8 / 12.9,
+// 14.1 / 13.7, 14.7 / 16.6; from 2^24 weights on the ring is ahead).
+bool lds_shape(int64_t N, int64_t K, bool fp8, int64_t cus) {
+    return (K <= 3 * kChunk && N <= kBlockRows * cus) || (!fp8 && small_layer(N, K));
+}
 
 // LDS above the 64 KB default needs the attribute, once per kernel instance.
 int allow_lds(const void* kern, size_t shmem, bool* done) {
@@ -995,9 +1011,10 @@ int launch_ring_mfma(const MfmaArgs& a, hipStream_t s) {
     r.K = a.K;
     r.part = a.part;
     r.epi = EPI;
-    // a kept call takes exactly the splits that hai_gemm_mfma_splits names, and so does the residual call that it
-    // equals bit for bit; the others, whose caller names no count, plan by the weight format
-    ring_plan(r, a.KSB, a.keep || (EPI == HAI_EPI_RESIDUAL && a.N <= kMaxResidualNormCols), device_cus());
+    // up to 8192 columns (where partials can be kept) every call takes the splits that hai_gemm_mfma_splits names,
+    // above it the plain ones plan by the weight format
+    const bool named = a.keep || a.N <= kMaxResidualNormCols;
+    ring_plan(r, named ? a.KSB : ring_splits(a.N, a.K, a.wq != nullptr, a.KSB, device_cus()), device_cus());
     const int rc = launch_ring(r, a.check, device_cus(), s);
     if (rc != HAI_OK || r.splits == 1 || a.keep) return rc;
     const int64_t n = static_cast<int64_t>(a.M) * ((a.N + 1) / 2);
@@ -1022,8 +1039,10 @@ bool use_dma(const MfmaArgs& a) {
 
 template <int EPI>
 int dispatch_mfma(const MfmaArgs& a, hipStream_t s) {
-    if (use_dma(a)) return a.M <= 32 ? launch_dma<2, EPI>(a, s) : launch_dma<4, EPI>(a, s);
-    if (ring_shape(a.M, a.K)) return launch_ring_mfma<EPI>(a, s);
+    if (!lds_shape(a.N, a.K, a.wq != nullptr, device_cus())) {
+        if (use_dma(a)) return a.M <= 32 ? launch_dma<2, EPI>(a, s) : launch_dma<4, EPI>(a, s);
+        if (ring_shape(a.M, a.K)) return launch_ring_mfma<EPI>(a, s);
+    }
     if (a.M <= 16) return launch_mfma<1, EPI>(a, s);
     if (a.M <= 32) return launch_mfma<2, EPI>(a, s);
     if (a.M <= 64) return launch_mfma<4, EPI>(a, s);
@@ -1042,13 +1061,6 @@ extern "C" size_t hai_gemm_mfma_workspace_bytes(int64_t M, int64_t N) {
 
 namespace {
 
-// K split across blocks for narrow layers (measured on MI355X at M = 32:
-// N = 5120 4 splits +115 %, N = 16384 2 splits +9 %), if the workspace holds
-// the partials and every split gets at least two chunks.  For N <= 8192 the
-// split count is the one that loads the busiest CU least (tiles x splits
-// blocks on the CUs, ties to more splits): the time of these launches
-// follows their busiest CU, so N = 5120 (80 tiles) takes 3 splits, 240
-// blocks, rather than 4, whose 320 blocks double up on 64 CUs.
 int device_cus() {
     static std::atomic<int> cached{0};  // one GPU model per process; retried until a device answers
     const int known = cached.load(std::memory_order_relaxed);
@@ -1062,24 +1074,26 @@ int device_cus() {
     return 256;  // MI355X
 }
 
+// K split across blocks for narrow layers (LDS-staged kernel, MI355X at M = 32:
+// N = 5120 4 splits +115 %, N = 16384 2 splits +9 %), if the workspace holds
+// the partials and every split gets at least two chunks.  For N <= 8192 the
+// split count is the ring's plan at FP8 prices (the caller of
+// hai_gemm_mfma_splits names no format) or, for small layers and shapes that the
+// ring does not take, the one that loads the busiest CU least (tiles x splits
+// blocks on the CUs): the time of these launches follows their busiest CU, so
+// N = 5120 (80 tiles) takes 3 splits, 240 blocks, rather than 4, whose 320 blocks
+// double up on 64 CUs.  Ties go to more splits, for the ring to fewer (taller
+// tiles cost it a chunk per step).
 int choose_splits(int64_t M, int64_t N, int64_t K, const void* workspace, size_t workspace_bytes) {
     const int64_t nck = (K + kChunk - 1) / kChunk;
     auto fits = [&](int64_t ksb) {
         return nck >= 2 * ksb && workspace != nullptr &&
                workspace_bytes >= static_cast<size_t>(ksb * M * N) * sizeof(float);
     };
-    if (N <= 8192 && ring_shape(M, K)) {
-        // the ring-staged kernel's plan, at FP8 prices: the caller of hai_gemm_mfma_splits names no format
-        static const float fp8_plan = 1.0f;
+    if (N <= 8192 && ring_shape(M, K) && !small_layer(N, K)) {
         int most = 4;
         while (most > 1 && !fits(most)) --most;
-        RingArgs r{};
-        r.scales = &fp8_plan;
-        r.M = static_cast<int>(M);
-        r.N = static_cast<int>(N);
-        r.K = static_cast<int>(K);
-        ring_plan(r, most, false, device_cus());
-        return r.splits;
+        return ring_splits(N, K, true, most, device_cus());
     }
     if (N <= 8192) {
         const int64_t cus = device_cus();
@@ -1089,7 +1103,7 @@ int choose_splits(int64_t M, int64_t N, int64_t K, const void* workspace, size_t
         for (int ksb = 2; ksb <= 4; ++ksb) {
             if (!fits(ksb) || ntiles * ksb > 2 * cus) continue;  // at most two blocks per CU
             const double load = static_cast<double>((ntiles * ksb + cus - 1) / cus) / ksb;
-            if (load <= best_load) {
+            if (load < best_load || (load == best_load && !ring_shape(M, K))) {
                 best = ksb;
                 best_load = load;
             }

@@ -27,9 +27,10 @@ struct RingArgs {
 constexpr int kRingK = 128;        // k per chunk (one FP8 scale block)
 constexpr int kRingMaxRows = 64;   // activation rows
 
-// Fills the plan: the tile height R and the K splits, up to max_splits (a
-// plane each in part), or exactly max_splits when fixed.
-void ring_plan(RingArgs& r, int max_splits, bool fixed, int cus);
+// The K splits of N x K weights, at most max_splits (a plane of part each).
+int ring_splits(int64_t N, int64_t K, bool fp8, int max_splits, int cus);
+// Fills the plan for `splits` splits: the tile height R.
+void ring_plan(RingArgs& r, int splits, int cus);
 // Needs K % kRingK == 0, M <= kRingMaxRows, 16-byte aligned x and w rows.
 // check: the codes may hold 0x7F / 0xFF.  With splits > 1 the partials are
 // left in part.

@@ -63,7 +63,7 @@ int ring_stages(int R, int mt, bool fp8, int kc) {
 // first copy (MI355X, one chunk per step / this, 8 rows FP8: 1024 x 1152 8.2 / 7.3
 // us, 5568 x 4992 14.2 / 12.8, 5568 x 8320 18.1 / 15.9; 32 rows: 5568 x 4992 14.7 /
 // 13.6, 14336 x 5248 22.7 / 23.8).
-int ring_kc(int R, int M, int K, bool fp8) { return M <= 32 && R <= (fp8 ? 96 : 64) && K >= 2 * kRingK ? 2 : 1; }
+int ring_kc(int R, int M, int64_t K, bool fp8) { return M <= 32 && R <= (fp8 ? 96 : 64) && K >= 2 * kRingK ? 2 : 1; }
 
 template <int MT, int NG, bool FP8, int KC>
 struct RingShape {
@@ -469,54 +469,70 @@ int launch_ring_ng(const RingArgs& r, int cus, hipStream_t s) {
 
 namespace hai {
 
-// The plan whose busiest CU copies the fewest bytes: the copies are what
-// bounds the kernel, weights (HBM) and activations (L2) alike, at 27-32 B per
-// ns and CU however many stages are in flight (MI355X, M = 64 FP8: gate|up,
-// 242 tiles of 144 rows, W alone 34 us, X alone 17, both 48).  A split adds its
-// partial planes and a second pass (about 9 us with its launch: 16384 x 5120 at
-// M = 64, 256 tiles of 64 33.5 us, 128 tiles of 128 in two splits 36.2).
-// Wide FP8 layers are not split into tiles too tall for two chunks per step
-// (more than 96 rows): MI355X, one / two splits at 8, 32 and 64 rows, 14336 x
-// 5120 19.9 / 21.6, 23.0 / 23.2, 28.5 / 29.9 us, 16480 x 5120 21.1 / 23.6, 24.4 /
-// 26.3, 32.5 / 33.6; where the tiles stay shorter two win, 12288 x 5120 20.3 / 17.7,
-// 22.5 / 19.7, 26.4 / 26.9.
-// The splits follow N, K, the weight format and the epilogue alone (priced for
-// 64 rows), so that a row's sums are the same whatever the number of rows: a
-// verify and a correction of the same row round alike.
-void ring_plan(RingArgs& r, int max_splits, bool fixed, int cus) {
-    const bool fp8 = r.scales != nullptr;
+namespace {
+// The tile height of N x K weights whose busiest CU copies the fewest bytes for
+// M rows and `splits` splits, and those bytes: the copies are what bounds the
+// kernel, weights (HBM) and activations (L2) alike, at 27-32 B per ns and CU
+// however many stages are in flight (MI355X, M = 64 FP8: gate|up, 242 tiles of
+// 144 rows, W alone 34 us, X alone 17, both 48).
+int best_tile(int M, int64_t N, int64_t K, bool fp8, int splits, int cus, double& cost) {
     const int eb = fp8 ? 1 : 2;
-    const int64_t nck = r.K / kRingK;
-    // the best tile height for `splits` splits of M rows, and its cost
-    auto best_tile = [&](int M, int splits, double& cost) {
-        const int mt = M <= 32 ? 1 : 2;
-        int best = 0;
-        for (int R = 32; R <= 160; R += 16) {
-            if (ring_stages(R, mt, fp8, ring_kc(R, M, r.K, fp8)) < 3) break;
-            const int64_t tiles = (static_cast<int64_t>(r.N) + R - 1) / R;
-            const int64_t rounds = (tiles * splits + cus - 1) / cus;
-            const double c = static_cast<double>(rounds) * static_cast<double>((nck + splits - 1) / splits) *
-                             (R * kRingK * eb + mt * 32 * kRingK * 2);
-            if (best == 0 || c < cost) {
-                best = R;
-                cost = c;
-            }
-        }
-        return best;
-    };
-    r.splits = max_splits;
-    double cost = 0.0;
-    for (int splits = 1; splits <= max_splits && !fixed; ++splits) {
-        double c = 0.0;
-        const int R = best_tile(kRingMaxRows, splits, c);
-        if (splits > 1 && fp8 && r.N > 8192 && ring_kc(R, 1, r.K, fp8) == 1) continue;
-        if (splits > 1) c += 270e3 + 8.0 * splits * kRingMaxRows * r.N / cus;
-        if (splits == 1 || c < cost) {
-            r.splits = splits;
+    const int mt = M <= 32 ? 1 : 2;
+    const int64_t nck = K / kRingK;
+    int best = 0;
+    for (int R = 32; R <= 160; R += 16) {
+        if (ring_stages(R, mt, fp8, ring_kc(R, M, K, fp8)) < 3) break;
+        const int64_t tiles = (N + R - 1) / R;
+        const int64_t rounds = (tiles * splits + cus - 1) / cus;
+        const double c = static_cast<double>(rounds) * static_cast<double>((nck + splits - 1) / splits) *
+                         (R * kRingK * eb + mt * 32 * kRingK * 2);
+        if (best == 0 || c < cost) {
+            best = R;
             cost = c;
         }
     }
-    r.R = best_tile(r.M, r.splits, cost);
+    return best;
+}
+}  // namespace
+
+// The splits follow N, K and the weight format alone (priced for 64 rows), so
+// that a row's sums are the same whatever the number of rows: a verify and a
+// correction of the same row round alike.  FP8 tiles too tall for two chunks per
+// step (more than 96 rows) are slower than their bytes.  Above 8192 columns they
+// are not taken: MI355X, one / two splits at 8, 32 and 64 rows, 14336 x 5120 FP8
+// 19.9 / 21.6, 23.0 / 23.2, 28.5 / 29.9 us, 16480 x 5120 21.1 / 23.6, 24.4 / 26.3, 32.5 /
+// 33.6; where the tiles stay shorter two win, 12288 x 5120 20.3 / 17.7, 22.5 / 19.7,
+// 26.4 / 26.9, for about 9 us of partial planes and second pass.  Up to 8192 the
+// shorter walk over K outweighs the second pass wherever the splits shorten it,
+// and tall tiles cost a step's worth: 1 / 2 / 3 / 4 splits at 8 and 64 rows FP8, 1024 x
+// 2944 15.1 / 10.7 / 9.2 / 8.7 and 20.1 / 13.2 / 11.5 / 10.7 us, 5120 x 4096 18.5 / 13.7 /
+// 12.5 / 12.1 and 24.4 / 16.6 / 15.8 / 16.2, 8192 x 4096 (tall from three on) 19.6 / 14.1 /
+// 15.1 / 14.9 and 24.7 / 17.2 / 19.8 / 19.7.  (Over 81 shapes of 512-8192 x 1024-6144 the
+// plan is 1-2 % behind the best split on average, 16 % at most; priced with 9 us
+// for the second pass it was 13 % behind, 84 % at most.)
+int ring_splits(int64_t N, int64_t K, bool fp8, int max_splits, int cus) {
+    int best = 1;
+    double cost = 0.0;
+    for (int splits = 1; splits <= max_splits; ++splits) {
+        double c = 0.0;
+        const int R = best_tile(kRingMaxRows, N, K, fp8, splits, cus, c);
+        if (splits > 1) {
+            const bool tall = fp8 && ring_kc(R, 1, K, fp8) == 1;
+            if (tall && N > 8192) continue;
+            c += (N > 8192 ? 270e3 : tall ? 150e3 : 0.0) + 8.0 * splits * kRingMaxRows * static_cast<double>(N) / cus;
+        }
+        if (splits == 1 || c < cost) {
+            best = splits;
+            cost = c;
+        }
+    }
+    return best;
+}
+
+void ring_plan(RingArgs& r, int splits, int cus) {
+    double cost = 0.0;
+    r.splits = splits;
+    r.R = best_tile(r.M, r.N, r.K, r.scales != nullptr, splits, cus, cost);
     r.tiles = (r.N + r.R - 1) / r.R;
 }
 
