@@ -2043,3 +2043,9 @@ def test_gemm_mfma_stream_k_matches_plain_grid(fp8, M, N, K, epi):
     # epilogue rounds acc before adding it: a regrouping flip compounds to a
     # few ulps of the operands, twice the one-sided oracle tolerance
     assert np.allclose(sk, plain, rtol=2 ** -6, atol=2 ** -8 * np.abs(plain).max()), float(np.abs(sk - plain).max())
+
+
+def test_gemm_fp8_mfma_stream_k():
+    """FP8 stream-K: K a multiple of 16 but not of 128 (the others up to 64
+    rows are the ring-staged kernel's)."""
+    test_gemm_mfma_stream_k_matches_plain_grid(True, 40, 33800, 5008, 1)
