@@ -1665,13 +1665,13 @@ def test_gemm_ring_rows_do_not_depend_on_the_row_count(fp8, N, K):
         assert np.array_equal(r, rows[0])
 
 
-@pytest.mark.parametrize("fp8,N,K,splits", [
-    (True, 5120, 3840, 4), (True, 5120, 11008, 4), (False, 4096, 4352, 4),  # K / 256 not a multiple of the splits
-    (True, 8192, 4992, 2),  # an odd number of 128-k chunks
-    (True, 14336, 5120, None), (True, 14336, 1024, None),  # wide layers: ring-staged without a split, copy-staged
-    (False, 1536, 2560, 4), (True, 1536, 2560, 4), (True, 5120, 2048, 3), (True, 9000, 768, 1),  # small layers
-    (False, 8192, 2176, 2)])
-def test_gemm_split_rows_do_not_depend_on_the_row_count(fp8, N, K, splits):
+@pytest.mark.parametrize("fp8,N,K,split", [
+    (True, 5120, 3840, True), (True, 5120, 11008, True), (False, 4096, 4352, True),  # K / 256 not a multiple of them
+    (True, 8192, 4992, True),  # an odd number of 128-k chunks
+    (True, 14336, 5120, False), (True, 14336, 1280, False),  # wide layers: ring-staged without a split, copy-staged
+    (False, 1536, 2560, True), (True, 1536, 2560, True), (True, 5120, 2048, True),  # small layers
+    (True, 9000, 768, False), (False, 8192, 1920, True)])
+def test_gemm_split_rows_do_not_depend_on_the_row_count(fp8, N, K, split):
     """A row gives the same bits whether the call has 4 or 64 rows (a verify
     and a correction of the same row round alike)."""
     rng = np.random.default_rng(N + K)
@@ -1687,8 +1687,8 @@ def test_gemm_split_rows_do_not_depend_on_the_row_count(fp8, N, K, splits):
         dy = out_buf(M * N * 2)
         wsb = kern().hai_gemm_mfma_workspace_bytes(M, N)
         dws = out_buf(max(wsb, 16))
-        if splits is not None:
-            assert kern().hai_gemm_mfma_splits(M, N, K, dws.ptr, wsb) == splits
+        if split:
+            assert kern().hai_gemm_mfma_splits(M, N, K, dws.ptr, wsb) > 1
         if fp8:
             hai.check(kern().hai_gemm_fp8_mfma(dy.ptr, N, dx.ptr, K, dw.ptr, ds.ptr, None, M, N, K,
                                                hai.FP8_NO_SPECIAL_CODES, None, 0, dws.ptr, wsb, None), "fp8 mfma")

@@ -876,15 +876,17 @@ bool ring_shape(int64_t M, int64_t K) { return K % kRingK == 0 && M <= kRingMaxR
 bool small_layer(int64_t N, int64_t K) { return N <= 8192 && K <= 8192 && N * K <= (int64_t{1} << 24); }
 
 // Of the ring's shapes, those that the LDS-staged kernel keeps, because its
-// blocks start faster: walks too short to be split, in at most one 64-row tile
-// per CU (MI355X, ring / LDS-staged at 4, 32 and 64 rows: 8192 x 512 FP8 6.1 / 4.9,
-// 9.9 / 5.9, 10.6 / 8.1 us, 16384 x 768 FP8 7.5 / 6.5, 8.8 / 7.9, 9.6 / 10.3, 12288 x 512
-// bf16 7.5 / 5.2, 10.7 / 6.0, 12.1 / 8.3; 34816 x 512 9.7 / 11.9, 12.9 / 16.2, 17.7 /
-// 16.9), and small bf16 layers (4, 32 and 64 rows: 1024 x 2944 10.6 / 8.5, 9.9 / 8.9,
-// 10.8 / 11.6, 4096 x 2048 11.4 / 9.0, 13.1 / 10.2, 15.2 / 12.2, 2048 x 6144 13.8 / 12.9,
-// 14.1 / 13.7, 14.7 / 16.6; from 2^24 weights on the ring is ahead).
+// blocks start faster: walks of at most four 256-k chunks, which are not split,
+// in at most one 64-row tile per CU (MI355X, ring / LDS-staged at 4, 32 and 64
+// rows: 8192 x 512 FP8 6.1 / 4.9, 9.9 / 5.9, 10.6 / 8.1 us, 16384 x 768 FP8 7.5 / 6.5,
+// 8.8 / 7.9, 9.6 / 10.3, 12288 x 512 bf16 7.5 / 5.2, 10.7 / 6.0, 12.1 / 8.3; at 8, 32 and 64
+// rows 5632 x 1024 FP8 7.8 / 6.8, 11.2 / 8.3, 12.8 / 11.1, bf16 8.8 / 6.1, 12.2 / 7.4, 12.8 /
+// 10.6; wider than a tile per CU 34816 x 512 FP8 9.4 / 12.1, 12.9 / 16.2, 17.7 / 16.9), and
+// small bf16 layers (8, 32 and 64 rows: 1024 x 2944 10.2 / 8.6, 9.9 / 8.9, 10.8 / 11.6,
+// 4096 x 2048 10.9 / 9.0, 13.1 / 10.2, 15.2 / 12.2, 2048 x 6144 13.8 / 12.9, 14.1 / 13.7,
+// 14.7 / 16.6; from 2^24 weights on the ring is ahead).
 bool lds_shape(int64_t N, int64_t K, bool fp8, int64_t cus) {
-    return (K <= 3 * kChunk && N <= kBlockRows * cus) || (!fp8 && small_layer(N, K));
+    return (K <= 4 * kChunk && N <= kBlockRows * cus) || (!fp8 && small_layer(N, K));
 }
 
 // LDS above the 64 KB default needs the attribute, once per kernel instance.
@@ -1076,7 +1078,9 @@ int device_cus() {
 
 // K split across blocks for narrow layers (LDS-staged kernel, MI355X at M = 32:
 // N = 5120 4 splits +115 %, N = 16384 2 splits +9 %), if the workspace holds
-// the partials and every split gets at least two chunks.  For N <= 8192 the
+// the partials and every split gets at least two chunks, three up to 64 rows:
+// two leave too little to outweigh the second launch (5632 x 1024 FP8 in two
+// splits 7.5 us at 8 rows, unsplit 6.8).  For N <= 8192 the
 // split count is the ring's plan at FP8 prices (the caller of
 // hai_gemm_mfma_splits names no format) or, for small layers and shapes that the
 // ring does not take, the one that loads the busiest CU least (tiles x splits
@@ -1086,8 +1090,9 @@ int device_cus() {
 // tiles cost it a chunk per step).
 int choose_splits(int64_t M, int64_t N, int64_t K, const void* workspace, size_t workspace_bytes) {
     const int64_t nck = (K + kChunk - 1) / kChunk;
+    const int64_t least = ring_shape(M, K) ? 3 : 2;  // chunks of a split
     auto fits = [&](int64_t ksb) {
-        return nck >= 2 * ksb && workspace != nullptr &&
+        return nck >= least * ksb && workspace != nullptr &&
                workspace_bytes >= static_cast<size_t>(ksb * M * N) * sizeof(float);
     };
     if (N <= 8192 && ring_shape(M, K) && !small_layer(N, K)) {
