@@ -99,3 +99,28 @@ def test_copy_staged_mfma_pipeline_waits(tmp_path):
             assert not stray, f"{m.group(1)}: {stray} between the pipeline wait and the reads"
         checked += 1
     assert checked >= 6, f"only {checked} copy-staged kernels found"
+
+
+def test_ring_kernels_use_no_scratch(tmp_path):
+    """gemm_ring_mfma_kernel (hai_gemm_ring.hip): no form keeps registers in
+    scratch memory.  The 12-wave forms are held to 168 registers; row offsets
+    formed ahead of the item loop would be spilled, and each reload's wait
+    would drain the activation copies of the next item."""
+    import build
+    if not Path(build.HIPCC).exists() and shutil.which("hipcc") is None:
+        pytest.skip("hipcc not available")
+    out = tmp_path / "ring.s"
+    flags = [f for f in build.HIP_FLAGS if f != "-fPIC"]
+    subprocess.run([build.HIPCC, *flags, "--cuda-device-only", "-S", str(build.CSRC / "hai_gemm_ring.hip"), "-o",
+                    str(out)], check=True, capture_output=True, timeout=900)
+    lines = out.read_text().split("\n")
+    checked = 0
+    for i, line in enumerate(lines):
+        m = re.match(r"^(_Z\S*gemm_ring_mfma_kernel\S*):", line)
+        if not m:
+            continue
+        end = next(j for j in range(i, len(lines)) if "s_endpgm" in lines[j])
+        stop = next(j for j in range(end, len(lines)) if lines[j].startswith(".Lfunc_end"))
+        assert not any("scratch_" in l for l in lines[i:stop]), f"{m.group(1)}: scratch memory"
+        checked += 1
+    assert checked >= 30, f"only {checked} ring-staged kernels found"

@@ -391,22 +391,28 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
         const int64_t n = static_cast<int64_t>(tile) * R + wrow;
         const bool col = wrow < R && n < a.N;
         const int m0 = 32 * mg + 4 * lh;
+        // the pitches are made opaque here, or the compiler forms the 16 row offsets before the item loop and spills them
+        // (27B MLP, 64 rows FP8: 89 -> 79 us)
+        int64_t ldy = a.ldy, ldres = a.ldres, pitch = a.N;
+        asm volatile("" : "+s"(ldy), "+s"(ldres), "+s"(pitch));
         if (a.splits > 1) {
             if (col) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const int m = m0 + 8 * (i >> 2) + (i & 3);
-                    if (m < a.M) a.part[(static_cast<int64_t>(split) * a.M + m) * a.N + n] = tot[i];
+                    if (m < a.M) a.part[(static_cast<int64_t>(split) * a.M + m) * pitch + n] = tot[i];
                 }
             }
         } else if (a.epi == HAI_EPI_SILU_MUL) {
+            // lanes lc, lc ^ 1 hold a gate and its up column: the even one takes elements 0 .. 7, the odd one 8 .. 15
+            const bool odd = (lc & 1) != 0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int m = m0 + 8 * (i >> 2) + (i & 3);
-                const float g = bfr(tot[i]);
-                const float u = quad_xor1(g);
-                if ((lc & 1) == 0 && col && m < a.M)
-                    a.y[static_cast<int64_t>(m) * a.ldy + n / 2] = f2bf(hw_silu(g) * u);
+            for (int i = 0; i < 8; ++i) {
+                const float a0 = bfr(tot[i]), a1 = bfr(tot[i + 8]);
+                const float b0 = quad_xor1(a0), b1 = quad_xor1(a1);
+                const int m = m0 + 8 * (i >> 2) + (i & 3) + (odd ? 16 : 0);
+                if (col && m < a.M)
+                    a.y[static_cast<int64_t>(m) * ldy + n / 2] = f2bf(hw_silu(odd ? b1 : a0) * (odd ? a1 : b0));
             }
         } else if (col) {
 #pragma unroll
@@ -414,8 +420,8 @@ __global__ __launch_bounds__(64 * (NG * MT + kRingCopiers)) void gemm_ring_mfma_
                 const int m = m0 + 8 * (i >> 2) + (i & 3);
                 if (m >= a.M) continue;
                 float o = bfr(tot[i]);
-                if (a.epi == HAI_EPI_RESIDUAL) o = bf2f(a.res[static_cast<int64_t>(m) * a.ldres + n]) + o;
-                a.y[static_cast<int64_t>(m) * a.ldy + n] = f2bf(o);
+                if (a.epi == HAI_EPI_RESIDUAL) o = bf2f(a.res[static_cast<int64_t>(m) * ldres + n]) + o;
+                a.y[static_cast<int64_t>(m) * ldy + n] = f2bf(o);
             }
         }
     }
