@@ -1256,14 +1256,15 @@ inline bool fa_enabled() {
 // The flash form reads every K / V tile once per 32 W query rows and needs
 // no merge pass, but a block walks its whole key range alone (2.8 us per 64
 // keys at D = 256), so it needs enough blocks; the split form spreads the
-// keys of few rows over the device.  Measured on MI355X (us, split / flash),
-// blocks counted at 256 rows: D = 256, 1 x 512 rows over 512 / 8192 keys (48
-// blocks) 52 / 38 and 405 / 348, 1 x 1024 over 1024 (96) 100 / 60, 4 x 1024
-// over 4096 (384) 1413 / 428, against 46 / 58 at 32 blocks; D = 128 76 / 117
-// at 24 blocks, 105 / 64 at 48, 433 / 231 at 128; D = 64 143 / 165 at 64,
-// 37 / 28 and 172 / 165 at 96.  Below half the CUs four-wave blocks (twice as
-// many) are 5-15 % faster; from there on eight waves are (2 x 1024 over 1024,
-// 192 blocks: 102 / 69), two per SIMD covering each other's softmax and LDS
+// keys of few rows over the device.  Measured on MI355X (us, split / flash,
+// norms and append included), blocks counted at 256 rows: D = 256, 1 x 512 rows
+// over 512 / 8192 keys (48 blocks) 61 / 48 and 415 / 314, 1 x 1024 over 1024 (96)
+// 113 / 72, 2 x 1024 over 1024 (192) 206 / 97, 4 x 1024 over 4096 (384) 1459 / 489;
+// D = 128 49 / 29 at 72 blocks, 826 / 292 at 192; D = 64 38 / 24 and 188 / 147 at 96;
+// below the lines (an earlier flash kernel, alone) 46 / 58 at 32 blocks of D = 256,
+// 76 / 117 at 24 of D = 128, 143 / 165 at 64 of D = 64.  Below half the CUs four-wave
+// blocks (twice as many) are 5-15 % faster; from there on eight waves are, two per
+// SIMD covering each other's softmax and LDS
 // latency.  128 rows at least: fewer leave the block's other rows idle.
 // The output and gate rows are accessed 8 bytes at a time.
 inline int fa_waves(int D, int64_t B, int64_t nqry, int64_t nkv, const void* out, const void* gate) {
