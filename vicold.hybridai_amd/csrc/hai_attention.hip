@@ -951,7 +951,7 @@ __global__ __launch_bounds__(256) void gqa_mfma_combine_wave_kernel(uint16_t* __
 //   S^T = K Q^T  on v_mfma_f32_32x32x16_bf16 (K rows the A operand from LDS,
 //                Q^T the B operand held in registers for the whole kernel);
 //   online softmax per query (base 2, P rounded to bf16, the running max moved
-//                past kFaRescaleSlack);
+//                past kFaRescaleSlack, later kFaLateSlack);
 //   O^T += V^T P^T  (the result tile of S^T is the B operand of this product
 //                as it stands, under the key order 4 lh + q % 4 + 8 (q / 4)
 //                of k slot q; V^T comes out of the V rows in LDS through the
@@ -972,7 +972,7 @@ __global__ __launch_bounds__(256) void gqa_mfma_combine_wave_kernel(uint16_t* __
 // keeps four-wave blocks, one wave per SIMD, to 256 registers as well: given 512
 // the compiler holds O in accumulation registers and rescales it through
 // moves (1 x 1024 rows over 1024 keys 84 -> 68 us with the norms).  MI355X, D =
-// 256, 8 x 1024 rows over 8192 keys, norms and append included: 3932 -> 1542 us
+// 256, 8 x 1024 rows over 8192 keys, norms and append included: 3932 -> 1534 us
 // against four waves of one per SIMD with V transposed through registers and
 // the copies' wait exposed.
 // ---------------------------------------------------------------------------
@@ -982,10 +982,13 @@ constexpr int kFaKeys = 64;      // keys per staged tile (two halves of 32)
 // because a row's heaviest weight is exact in bf16 when it is the reference
 // itself, and rounded like any other under an older one (by up to 2^slack).
 // MI355X, error against float64 of 1024 rows over 1024 keys / time of 8 x 1024
-// rows over 8192: 0 2.923e-3 / 1553 us, 1/8 2.930e-3 / 1542, 1/4 2.934e-3 / 1520,
-// 1 2.946e-3 / 1506, 8 2.972e-3 / 1490; the split form's waves, each with a
-// reference of its own, have 2.943e-3.
-constexpr float kFaRescaleSlack = 0.125f;
+// rows over 8192, one slack throughout: 0 2.923e-3 / 1553 us, 1/8 2.930e-3 / 1542, 1
+// 2.946e-3 / 1506, 8 2.972e-3 / 1490; the split form's waves, each with a reference
+// of its own, have 2.943e-3.  Past the first kFaLateKeys keys a larger maximum is
+// rare and shares its row with many weights, and the slack is wider: 8 x 1024 rows
+// over 8192 keys 2.877e-3 -> 2.890e-3 (split form 2.911e-3) and 2 % of the time back.
+constexpr float kFaRescaleSlack = 0.125f, kFaLateSlack = 1.0f;
+constexpr int kFaLateKeys = 1024;
 
 template <int D>
 struct FaShape {
@@ -1160,7 +1163,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void gqa_fa_kernel(uint16_t* __restr
 #pragma unroll
             for (int i = 2; i < 16; ++i) mx = fmaxf(mx, st[i]);
             mx = fmaxf(mx, __shfl_xor(mx, 32)) * scale_log2;
-            const bool grow = mx > m + kFaRescaleSlack;  // true for the first visible key
+            const bool grow = mx > m + (k0 < kFaLateKeys ? kFaRescaleSlack : kFaLateSlack);  // true for the first visible key
             if (__builtin_amdgcn_ballot_w64(grow) != 0) {
                 const float mn = grow ? mx : m;
                 const float alpha = grow ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;  // 0 from -inf
